@@ -71,6 +71,12 @@ int wl_dequant(int type, const void* w, int64_t rows, int64_t k, int64_t row_str
 int wl_gemv(int type, const void* w, int64_t rows, int64_t k, int64_t row_stride, const float* x, int64_t tokens,
             float* y, void* stream);
 
+/* wl_gemv with x and y each fp32 or bf16 (WL_DTYPE_*): bf16 values of x are read as they are, y is the fp32 sum
+ * rounded to nearest even when it is bf16. What the Metal gemv takes and returns (gguf/metal.py:189-215,327-334),
+ * without a conversion pass on either side. */
+int wl_gemv_dtype(int type, const void* w, int64_t rows, int64_t k, int64_t row_stride, const void* x, int x_dtype,
+                  int64_t tokens, void* y, int y_dtype, void* stream);
+
 /* y[t, r] = sum_k W[r, k] * x[t, k] for t < tokens on the bf16 matrix core: x bf16 [tokens x k] (row stride k),
  * W's exact values rounded to bf16 in registers (never written out), fp32 accumulation, y bf16 [tokens x rows].
  * rows and k multiples of 256; W dense rows (row stride = wl_row_bytes(type, k)), 16-byte aligned for Q4_K.

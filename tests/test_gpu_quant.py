@@ -67,6 +67,32 @@ def test_gemv_shapes(hip, name, rows, k, tokens):
     assert moe_ref.rel_err(got, expect) < TOL
 
 
+@pytest.mark.parametrize("name,rows,k", [
+    ("Q4_K", 1, 256), ("Q6_K", 37, 512), ("Q4_K", 130, 768), ("Q6_K", 31, 1024), ("Q4_K", 97, 2048),
+    ("Q6_K", 65, 2560), ("Q4_K", 33, 4096), ("Q6_K", 21, 6400), ("Q4_K", 4201, 2048), ("Q6_K", 16500, 2048)])
+@pytest.mark.parametrize("tokens", [1, 2, 7, 8])
+def test_gemv_forms(hip, name, rows, k, tokens):
+    """Every split of the GEMV (blocks per row 1 .. 25 over lanes, wavefronts and the K loop; 1, 2 and 4 rows per lane
+    group; a last workgroup with missing rows) in fp32, and bf16 in and out: the kernel's fp32 sums on the same values,
+    rounded once. Bound: 2 roundings per product and add of the longest chain (under 64 of them, errors of either sign)
+    over sum |w x|, and bf16's half ulp."""
+    rng = np.random.default_rng(rows + 3 * k + tokens)
+    w = synth.matrix(rng, name, rows, k)
+    w64 = q.dequantize_matrix(w, name, rows, k).astype(np.float64)
+    xb = torch.from_numpy(rng.standard_normal((tokens, k)).astype(np.float32)).to(torch.bfloat16)
+    x64 = xb.double().numpy()
+    expect, size = x64 @ w64.T, np.abs(x64) @ np.abs(w64).T
+    # the runs' unsigned form (a * q, b apart) makes terms up to a few times |w x|
+    bound = 64 * 2.0 ** -24 * 4 * size + 1e-30
+    raw = dev(w).reshape(-1)
+    got = hip.gemv(raw, name, (rows, k), xb.cuda().float())
+    assert (np.abs(got.cpu().double().numpy() - expect) <= bound).all()
+    y = F.linear(xb.cuda(), hip.GGMLWeight(raw, name, (rows, k)))
+    assert y.dtype == torch.bfloat16 and torch.equal(y, got.to(torch.bfloat16))
+    odd = torch.empty(tokens * k + 1, dtype=torch.bfloat16, device="cuda")[1:].view(tokens, k).copy_(xb)
+    assert torch.equal(F.linear(odd, hip.GGMLWeight(raw, name, (rows, k))), y)  # x off a 16-byte boundary
+
+
 def test_gemv_batch_and_combine(hip):
     """gate_up of 4 experts in one launch (gemv_batch), then down + weighted sum (gemv_combine), as
     Engine.batched_decode_experts drives them (engines/base.py:492-532)."""

@@ -1,0 +1,267 @@
+// Quantized matrix times a few tokens: y[t, r] = W[r, :] . x[t, :] (wl_gemv, wl_gemv_dtype). Replaces the Metal kernel
+// gemv_<T> (gguf/metal.py:189-215).
+#include <hip/hip_runtime.h>
+
+#include "wl_common.h"
+#include "wl_host.h"
+
+namespace wl {
+
+// A lane's two 16-value runs of a block as f16 pairs (values 0 and 2 of each packed word in e, 1 and 3 in o) whose
+// exponent bits are zero: v_fma_mix_f32 reads such a half as the subnormal q 2^-s, so no value is ever converted. The
+// pairs are made once per block and used for every token; a (the run's scale) carries the 2^s back, exactly.
+template <int TYPE>
+struct HalfRuns {
+    uint32_t e_lo[4], o_lo[4], e_hi[4], o_hi[4];
+    float a_lo, a_hi, b_lo, b_hi;
+    __device__ __forceinline__ void set(const RawLane<TYPE>& raw, int c) {
+        Lane32 l;
+        if constexpr (TYPE == WL_TYPE_Q4_K) {
+            raw.unpack_mix(c, l);
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                e_lo[i] = l.lo[i] & 0x000F000Fu;
+                o_lo[i] = (l.lo[i] >> 8) & 0x000F000Fu;
+                e_hi[i] = l.lo[i] & 0x00F000F0u;
+                o_hi[i] = (l.lo[i] >> 8) & 0x00F000F0u;
+            }
+            a_lo = l.a_lo;
+            a_hi = l.a_hi;
+        } else {
+            raw.unpack(c, l);
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                e_lo[i] = l.lo[i] & 0x00FF00FFu;
+                o_lo[i] = (l.lo[i] >> 8) & 0x00FF00FFu;
+                e_hi[i] = l.hi[i] & 0x00FF00FFu;
+                o_hi[i] = (l.hi[i] >> 8) & 0x00FF00FFu;
+            }
+            a_lo = l.a_lo * 16777216.0f;
+            a_hi = l.a_hi * 16777216.0f;
+        }
+        b_lo = l.b_lo;
+        b_hi = l.b_hi;
+    }
+    static __device__ __forceinline__ float dot(const uint32_t (&e)[4], const uint32_t (&o)[4], const float4 (&x)[4]) {
+        float s0 = 0.0f, s1 = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const wl_f16x2 he = __builtin_bit_cast(wl_f16x2, e[i]), ho = __builtin_bit_cast(wl_f16x2, o[i]);
+            s0 = __builtin_fmaf(static_cast<float>(he.x), x[i].x, s0);
+            s1 = __builtin_fmaf(static_cast<float>(ho.x), x[i].y, s1);
+            s0 = __builtin_fmaf(static_cast<float>(he.y), x[i].z, s0);
+            s1 = __builtin_fmaf(static_cast<float>(ho.y), x[i].w, s1);
+        }
+        return s0 + s1;
+    }
+    // the lane's share of the block's product with x (its two runs, their sums known)
+    __device__ __forceinline__ float run(const float4 (&xl)[4], const float4 (&xh)[4], float sxl, float sxh) const {
+        return a_lo * dot(e_lo, o_lo, xl) + b_lo * sxl + a_hi * dot(e_hi, o_hi, xh) + b_hi * sxh;
+    }
+};
+
+__device__ __forceinline__ void load_run16(const float* __restrict__ p, float4 (&x)[4]) { load_run(p, x); }
+__device__ __forceinline__ void load_run16(const uint16_t* __restrict__ p, float4 (&x)[4]) {
+    const uint4* q = reinterpret_cast<const uint4*>(p);
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const uint4 v = q[i];
+        x[2 * i] = make_float4(__builtin_bit_cast(float, v.x << 16), __builtin_bit_cast(float, v.x & 0xFFFF0000u),
+                               __builtin_bit_cast(float, v.y << 16), __builtin_bit_cast(float, v.y & 0xFFFF0000u));
+        x[2 * i + 1] = make_float4(__builtin_bit_cast(float, v.z << 16), __builtin_bit_cast(float, v.z & 0xFFFF0000u),
+                                   __builtin_bit_cast(float, v.w << 16), __builtin_bit_cast(float, v.w & 0xFFFF0000u));
+    }
+}
+
+// a summed over lanes l and l ^ 32 in the low half of the wavefront, b in the high half: one swap and one add for
+// two values (swap_add spends them on one)
+__device__ __forceinline__ float pair_add32(float a, float b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b),
+                                                    false, false);
+    return __builtin_bit_cast(float, static_cast<uint32_t>(r[0])) +
+           __builtin_bit_cast(float, static_cast<uint32_t>(r[1]));
+}
+// the same over lanes l and l ^ 16: a in the even rows of 16 lanes, b in the odd ones
+__device__ __forceinline__ float pair_add16(float a, float b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b),
+                                                    false, false);
+    return __builtin_bit_cast(float, static_cast<uint32_t>(r[0])) +
+           __builtin_bit_cast(float, static_cast<uint32_t>(r[1]));
+}
+
+// The matrix times TT tokens (1 .. 8). A block belongs to 8 lanes (wl_common.h), 2^ks blocks of a row to a wavefront
+// pass; a wavefront holds R rows in each of its 8 >> ks lane groups, and kw of the workgroup's 4 wavefronts split K
+// (their sums are added in LDS in a fixed order). The lane's x runs come straight from global memory (L2 and L1 hold
+// them) and serve R rows each.
+// What bounds it: at 8 tokens the products (8 FMAs per weight; Q6_K 2048 x 4096: 4,100 VALU cycles per SIMD = 1.7 us)
+// and the x reads, which are why a lane group holds several rows; at one token the launch and one trip to memory.
+// Measured per call in a graph (bf16 in and out; before: a row per wavefront, its x read again for every row, and a
+// converting launch on each side): Q4_K 4096 x 2048 at 1 token 8.2 -> 4.1 us, 8 tokens 21.5 -> 8.5; Q6_K 2048 x 4096
+// 9.3 -> 4.4 and 22.0 -> 8.7; Q4_K 2048 x 512 6.2 -> 2.9 and 10.1 -> 5.3.
+template <int TYPE, int TT, int R, typename XT>
+__global__ __launch_bounds__(256) void k_gemv(const uint8_t* __restrict__ w, int rows, int nb, int64_t row_stride,
+                                              const XT* __restrict__ x, int64_t ldx, void* __restrict__ y,
+                                              int64_t ldy, int y_bf16, int ks, int kw) {
+    constexpr int N = TT * R;
+    __shared__ float part[4][8 * N];  // [wavefront][(t R + r) subs + sub]
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int g = lane >> 3, c = lane & 7;
+    const int slot = g & ((1 << ks) - 1), sub = g >> ks, subs = 8 >> ks;
+    const int kwi = wv % kw, rset = wv / kw;
+    const int rows_wave = subs * R, rows_wg = 4 / kw * rows_wave;
+    const int wg_row0 = static_cast<int>(blockIdx.x) * rows_wg;
+    const int row0 = wg_row0 + rset * rows_wave + sub * R;
+    const int lo_start = BlockInfo<TYPE>::lo_start(c);
+    const uint8_t* rp[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) rp[r] = w + static_cast<int64_t>(min(row0 + r, rows - 1)) * row_stride;
+    float acc[N];
+#pragma unroll
+    for (int n = 0; n < N; n++) acc[n] = 0.0f;
+    for (int kb = (kwi << ks) + slot; kb < nb; kb += kw << ks) {
+        RawLane<TYPE> raw[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) raw[r].fetch(rp[r] + static_cast<int64_t>(kb) * BlockInfo<TYPE>::bytes, c);
+        const XT* xk = x + kb * kQK + lo_start;
+        HalfRuns<TYPE> h[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) h[r].set(raw[r], c);
+#pragma unroll
+        for (int t = 0; t < TT; t++) {
+            float4 xl[4], xh[4];
+            load_run16(xk + t * ldx, xl);
+            load_run16(xk + t * ldx + BlockInfo<TYPE>::hi_offset, xh);
+            const float sxl = sum16(xl), sxh = sum16(xh);
+#pragma unroll
+            for (int r = 0; r < R; r++) acc[t * R + r] += h[r].run(xl, xh, sxl, sxh);
+        }
+    }
+    if (ks == 3) {
+        // over all 64 lanes: the first two steps halve the number of values, and row q of 16 lanes ends with value
+        // 4 i + (q >> 1) + 2 (q & 1) of quadruple i
+        float u[(N + 1) / 2], v[(N + 3) / 4];
+#pragma unroll
+        for (int i = 0; i < (N + 1) / 2; i++) u[i] = pair_add32(acc[2 * i], acc[2 * i + 1 < N ? 2 * i + 1 : 2 * i]);
+#pragma unroll
+        for (int i = 0; i < (N + 3) / 4; i++)
+            v[i] = group_sum<16>(pair_add16(u[2 * i], u[2 * i + 1 < (N + 1) / 2 ? 2 * i + 1 : 2 * i]));
+        const int q = lane >> 4, at = (q >> 1) + 2 * (q & 1);
+        if ((lane & 15) == 0) {
+#pragma unroll
+            for (int i = 0; i < (N + 3) / 4; i++)
+                if (4 * i + at < N) part[wv][4 * i + at] = v[i];
+        }
+    } else {
+#pragma unroll
+        for (int n = 0; n < N; n++) {
+            float s = group_sum<8>(acc[n]);
+            if (ks >= 1) s += dpp<0x140>(s);
+            if (ks >= 2) s = swap_add<16>(s);
+            if ((lane & ((8 << ks) - 1)) == 0) part[wv][n * subs + sub] = s;
+        }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < TT * rows_wg; i += 256) {
+        const int t = i / rows_wg, rr = i - t * rows_wg, row = wg_row0 + rr;
+        if (row >= rows) continue;
+        const int rs = rr / rows_wave, in = rr - rs * rows_wave;
+        const int at = (t * R + in % R) * subs + in / R;
+        float s = part[rs * kw][at];
+        for (int j = 1; j < kw; j++) s += part[rs * kw + j][at];
+        if (y_bf16)
+            static_cast<uint16_t*>(y)[t * ldy + row] = static_cast<uint16_t>(f32_to_bf16_bits(s));
+        else
+            static_cast<float*>(y)[t * ldy + row] = s;
+    }
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// Host side
+
+struct GemvCall {
+    const uint8_t* w;
+    int rows, nb;
+    int64_t row_stride;
+    int64_t k;
+    int y_bf16;
+    hipStream_t s;
+};
+
+template <int TYPE, int TT, int R, typename XT>
+static void launch_gemv_r(const GemvCall& g, const XT* x, void* y, int ks, int kw) {
+    const int rows_wg = 4 / kw * (8 >> ks) * R;
+    const unsigned grid = static_cast<unsigned>((g.rows + rows_wg - 1) / rows_wg);
+    k_gemv<TYPE, TT, R, XT><<<grid, 256, 0, g.s>>>(g.w, g.rows, g.nb, g.row_stride, x, g.k, y, g.rows, g.y_bf16, ks,
+                                                   kw);
+}
+
+template <int TYPE, int TT, typename XT>
+static void launch_gemv_t(const GemvCall& g, const XT* x, void* y) {
+    const int ks = g.nb >= 8 ? 3 : g.nb >= 4 ? 2 : g.nb >= 2 ? 1 : 0;
+    const int kw = g.nb <= 8 ? 1 : g.nb <= 16 ? 2 : 4;
+    const int per_r = 4 / kw * (8 >> ks);  // rows of a workgroup per R
+    // rows per lane group: more reuse each x read, fewer leave more workgroups. From 512 workgroups on (1024 for one
+    // token, whose x reads are few) more rows win (us with 1 / 2 / 4 rows; Q6_K 8192 x 2048, 8 tokens 17.5 / 15.0 /
+    // 13.0, 1 token 7.0 / 6.4 / 7.0; Q6_K 2048 x 4096, 8 tokens 10.3 / 8.7 / 9.3); with fewer the launch is too thin
+    // (Q4_K 1024 x 2048, 8 tokens 5.6 / 6.4 / 7.8)
+    const int64_t least = TT == 1 ? 1024 : 512;
+    const int want = g.rows >= 4 * per_r * least ? 4 : g.rows >= 2 * per_r * least ? 2 : 1;
+    if (want == 4)
+        launch_gemv_r<TYPE, TT, 4>(g, x, y, ks, kw);
+    else if (want == 2)
+        launch_gemv_r<TYPE, TT, 2>(g, x, y, ks, kw);
+    else
+        launch_gemv_r<TYPE, TT, 1>(g, x, y, ks, kw);
+}
+
+template <int TYPE, typename XT>
+static void launch_gemv(const GemvCall& g, const XT* x, int64_t tokens, void* y) {
+    for (int64_t t0 = 0; t0 < tokens; t0 += 8) {
+        const XT* xt = x + t0 * g.k;
+        void* yt = static_cast<char*>(y) + t0 * g.rows * (g.y_bf16 ? 2 : 4);
+        switch (tokens - t0 < 8 ? tokens - t0 : 8) {
+            case 1: launch_gemv_t<TYPE, 1>(g, xt, yt); break;
+            case 2: launch_gemv_t<TYPE, 2>(g, xt, yt); break;
+            case 3: launch_gemv_t<TYPE, 3>(g, xt, yt); break;
+            case 4: launch_gemv_t<TYPE, 4>(g, xt, yt); break;
+            case 5: launch_gemv_t<TYPE, 5>(g, xt, yt); break;
+            case 6: launch_gemv_t<TYPE, 6>(g, xt, yt); break;
+            case 7: launch_gemv_t<TYPE, 7>(g, xt, yt); break;
+            default: launch_gemv_t<TYPE, 8>(g, xt, yt); break;
+        }
+    }
+}
+
+}  // namespace wl
+
+using namespace wl;
+
+extern "C" {
+
+int wl_gemv_dtype(int type, const void* w, int64_t rows, int64_t k, int64_t row_stride, const void* x, int x_dtype,
+                  int64_t tokens, void* y, int y_dtype, void* stream) {
+    const int rc = check_matrix(type, w, rows, k, row_stride);
+    if (rc) return rc;
+    if (!x || !y) return WL_EINVAL_NULL;
+    if (tokens <= 0) return WL_EINVAL_SHAPE;
+    if ((x_dtype != WL_DTYPE_F32 && x_dtype != WL_DTYPE_BF16) || (y_dtype != WL_DTYPE_F32 && y_dtype != WL_DTYPE_BF16))
+        return WL_EINVAL_DTYPE;
+    if (reinterpret_cast<uintptr_t>(x) % 16 != 0) return WL_EINVAL_ALIGN;
+    const GemvCall g{static_cast<const uint8_t*>(w), static_cast<int>(rows), static_cast<int>(k / kQK), row_stride, k,
+                     y_dtype == WL_DTYPE_BF16 ? 1 : 0, static_cast<hipStream_t>(stream)};
+    if (x_dtype == WL_DTYPE_BF16) {
+        const uint16_t* xb = static_cast<const uint16_t*>(x);
+        type == WL_TYPE_Q4_K ? launch_gemv<WL_TYPE_Q4_K>(g, xb, tokens, y) : launch_gemv<WL_TYPE_Q6_K>(g, xb, tokens, y);
+    } else {
+        const float* xf = static_cast<const float*>(x);
+        type == WL_TYPE_Q4_K ? launch_gemv<WL_TYPE_Q4_K>(g, xf, tokens, y) : launch_gemv<WL_TYPE_Q6_K>(g, xf, tokens, y);
+    }
+    return launch_status();
+}
+
+int wl_gemv(int type, const void* w, int64_t rows, int64_t k, int64_t row_stride, const float* x, int64_t tokens,
+            float* y, void* stream) {
+    return wl_gemv_dtype(type, w, rows, k, row_stride, x, WL_DTYPE_F32, tokens, y, WL_DTYPE_F32, stream);
+}
+
+}  // extern "C"

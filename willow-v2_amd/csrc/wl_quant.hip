@@ -1,5 +1,5 @@
-// Q4_K / Q6_K dequantization and GEMV kernels, and their C-ABI entry points (include/willow_hip.h).
-// Replaces the Metal kernels dequant_<T>, gemv_<T>, gemv_batch_<T>, gemv_combine_<T> (gguf/metal.py:189-291).
+// Q4_K / Q6_K dequantization and batched-expert GEMV kernels, and their C-ABI entry points (include/willow_hip.h).
+// Replaces the Metal kernels dequant_<T>, gemv_batch_<T>, gemv_combine_<T> (gguf/metal.py:217-291).
 #include <hip/hip_runtime.h>
 
 #include "wl_common.h"
@@ -63,51 +63,6 @@ __global__ __launch_bounds__(256) void k_dequant(const uint8_t* __restrict__ w, 
 template <int WIDTH>
 __device__ __forceinline__ float wsum(float v) {
     return group_sum<WIDTH>(v);
-}
-
-// y[t, r] = W[r, :] . x[t, :] for t < T <= TT.
-template <int TYPE, int TT, int WIDTH>
-__global__ __launch_bounds__(256) void k_gemv(const uint8_t* __restrict__ w, int rows, int nb, int64_t row_stride,
-                                              const float* __restrict__ x, int T, int64_t ldx,
-                                              float* __restrict__ y, int64_t ldy) {
-    constexpr int R = WIDTH == 64 ? 1 : 64 / WIDTH;
-    const int lane = threadIdx.x & 63;
-    const int wave = static_cast<int>((static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) >> 6);
-    const int nwaves = static_cast<int>((static_cast<int64_t>(gridDim.x) * blockDim.x) >> 6);
-    const int g = lane >> 3, c = lane & 7;
-    const int row_off = R > 1 ? g / nb : 0;
-    const int kb0 = R > 1 ? g % nb : g;
-    const int kb_step = R > 1 ? nb : 8;
-    const bool slot_used = R > 1 ? (g < R * nb) : true;
-    const int lo_start = BlockInfo<TYPE>::lo_start(c), hi_off = BlockInfo<TYPE>::hi_offset;
-    for (int r0 = wave * R; r0 < rows; r0 += nwaves * R) {
-        const int row = r0 + row_off;
-        float acc[TT];
-#pragma unroll
-        for (int t = 0; t < TT; t++) acc[t] = 0.0f;
-        if (slot_used && row < rows) {
-            const uint8_t* rp = w + static_cast<int64_t>(row) * row_stride;
-            for (int kb = kb0; kb < nb; kb += kb_step) {
-                Lane32 l;
-                decode<TYPE>(rp + static_cast<int64_t>(kb) * BlockInfo<TYPE>::bytes, c, l);
-                const int lo = kb * kQK + lo_start;
-#pragma unroll
-                for (int t = 0; t < TT; t++) {
-                    if (t < T) {
-                        float4 xl[4], xh[4];
-                        load_run(x + t * ldx + lo, xl);
-                        load_run(x + t * ldx + lo + hi_off, xh);
-                        acc[t] += lane_dot(l, xl, xh);
-                    }
-                }
-            }
-        }
-#pragma unroll
-        for (int t = 0; t < TT; t++) {
-            const float s = wsum<WIDTH>(acc[t]);
-            if (t < T && (lane & (WIDTH - 1)) == 0 && row < rows) y[t * ldy + row] = s;
-        }
-    }
 }
 
 // Batched experts, one token: grid.y = expert i; y[pos[i], r] = W_i[r, :] . x.
@@ -198,37 +153,6 @@ __global__ __launch_bounds__(256) void k_gemv_combine(const uint8_t* __restrict_
 
 static int blocks_for_waves(int64_t waves) { return static_cast<int>((waves + 3) / 4); }
 
-template <int TYPE, int TT>
-static void launch_gemv_tt(const uint8_t* w, int rows, int nb, int64_t row_stride, const float* x, int T,
-                           int64_t ldx, float* y, int64_t ldy, hipStream_t s) {
-    const RowGeom geo = row_geom(nb);
-    const int grid = blocks_for_waves((rows + geo.R - 1) / geo.R);
-    switch (geo.width) {
-        case 8: k_gemv<TYPE, TT, 8><<<grid, 256, 0, s>>>(w, rows, nb, row_stride, x, T, ldx, y, ldy); break;
-        case 16: k_gemv<TYPE, TT, 16><<<grid, 256, 0, s>>>(w, rows, nb, row_stride, x, T, ldx, y, ldy); break;
-        case 32: k_gemv<TYPE, TT, 32><<<grid, 256, 0, s>>>(w, rows, nb, row_stride, x, T, ldx, y, ldy); break;
-        default: k_gemv<TYPE, TT, 64><<<grid, 256, 0, s>>>(w, rows, nb, row_stride, x, T, ldx, y, ldy); break;
-    }
-}
-
-template <int TYPE>
-static void launch_gemv(const uint8_t* w, int rows, int nb, int64_t row_stride, const float* x, int64_t tokens,
-                        int64_t k, float* y, hipStream_t s) {
-    for (int64_t t0 = 0; t0 < tokens; t0 += 8) {
-        const int T = static_cast<int>(tokens - t0 < 8 ? tokens - t0 : 8);
-        const float* xt = x + t0 * k;
-        float* yt = y + t0 * rows;
-        if (T == 1)
-            launch_gemv_tt<TYPE, 1>(w, rows, nb, row_stride, xt, T, k, yt, rows, s);
-        else if (T == 2)
-            launch_gemv_tt<TYPE, 2>(w, rows, nb, row_stride, xt, T, k, yt, rows, s);
-        else if (T <= 4)
-            launch_gemv_tt<TYPE, 4>(w, rows, nb, row_stride, xt, T, k, yt, rows, s);
-        else
-            launch_gemv_tt<TYPE, 8>(w, rows, nb, row_stride, xt, T, k, yt, rows, s);
-    }
-}
-
 template <int TYPE>
 static void launch_gemv_batch(const uint8_t* base, int rows, int nb, int64_t row_stride, const float* x,
                               float* out, const BatchTable& tab, int n, hipStream_t s) {
@@ -300,23 +224,6 @@ int wl_dequant(int type, const void* w, int64_t rows, int64_t k, int64_t row_str
         else
             k_dequant<WL_TYPE_Q6_K, false><<<grid, 256, 0, s>>>(wb, rows, nb, row_stride, out);
     }
-    return launch_status();
-}
-
-int wl_gemv(int type, const void* w, int64_t rows, int64_t k, int64_t row_stride, const float* x, int64_t tokens,
-            float* y, void* stream) {
-    int rc = check_matrix(type, w, rows, k, row_stride);
-    if (rc) return rc;
-    if (!x || !y) return WL_EINVAL_NULL;
-    if (tokens <= 0) return WL_EINVAL_SHAPE;
-    if (reinterpret_cast<uintptr_t>(x) % 16 != 0) return WL_EINVAL_ALIGN;
-    const int nb = static_cast<int>(k / kQK);
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    const uint8_t* wb = static_cast<const uint8_t*>(w);
-    if (type == WL_TYPE_Q4_K)
-        launch_gemv<WL_TYPE_Q4_K>(wb, static_cast<int>(rows), nb, row_stride, x, tokens, k, y, s);
-    else
-        launch_gemv<WL_TYPE_Q6_K>(wb, static_cast<int>(rows), nb, row_stride, x, tokens, k, y, s);
     return launch_status();
 }
 

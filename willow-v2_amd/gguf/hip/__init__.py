@@ -71,6 +71,7 @@ def library() -> ctypes.CDLL:
     lib.wl_row_bytes.argtypes, lib.wl_row_bytes.restype = [c_int, i64], i64
     lib.wl_dequant.argtypes = [c_int, vp, i64, i64, i64, c_int, vp, vp]
     lib.wl_gemv.argtypes = [c_int, vp, i64, i64, i64, vp, i64, vp, vp]
+    lib.wl_gemv_dtype.argtypes = [c_int, vp, i64, i64, i64, vp, c_int, i64, vp, c_int, vp]
     lib.wl_linear.argtypes = [c_int, vp, i64, i64, vp, i64, vp, vp]
     lib.wl_gemv_batch.argtypes = [c_int, vp, i64, i64, i64p, i64p, c_int, vp, vp, vp]
     lib.wl_gemv_combine.argtypes = [c_int, vp, i64, i64, i64p, i64p, c_int, vp, vp, vp, vp]
@@ -89,8 +90,8 @@ def library() -> ctypes.CDLL:
     lib.wl_moe_workspace_status.argtypes, lib.wl_moe_workspace_status.restype = [vp, ctypes.c_size_t, vp], c_int
     lib.wl_moe_fork_begin.argtypes, lib.wl_moe_fork_begin.restype = [vp], c_int
     lib.wl_moe_fork_end.argtypes, lib.wl_moe_fork_end.restype = [vp], c_int
-    for name in ("wl_dequant", "wl_gemv", "wl_linear", "wl_gemv_batch", "wl_gemv_combine", "wl_moe_check", "wl_moe_route",
-                 "wl_moe_layer", "wl_moe_layer_profile"):
+    for name in ("wl_dequant", "wl_gemv", "wl_gemv_dtype", "wl_linear", "wl_gemv_batch", "wl_gemv_combine", "wl_moe_check",
+                 "wl_moe_route", "wl_moe_layer", "wl_moe_layer_profile"):
         getattr(lib, name).restype = c_int
     _lib = lib
     return lib
@@ -295,11 +296,27 @@ class GGMLWeight:
         """Frees the kept bf16 values (the next call above MAX_TOKENS with keep_dense dequantizes again)."""
         self._dense = None
 
+    def _gemv_bf16(self, x: torch.Tensor) -> torch.Tensor:
+        """gemv(x).to(bf16) for bf16 x in one launch: the kernel reads bf16 and rounds its fp32 sums on the way out
+        (a converting launch on either side of it took as long as the GEMV itself)."""
+        rows, k = self.shape
+        x = x.reshape(-1, k).contiguous()
+        if x.data_ptr() % 16:  # a view that starts off a 16-byte boundary
+            x = x.clone()
+        y = torch.empty(x.shape[0], rows, dtype=torch.bfloat16, device=self.raw.device)
+        check(library().wl_gemv_dtype(TYPE_IDS[self.type_name], self.raw.data_ptr(), rows, k,
+                                      row_bytes(self.type_name, k), x.data_ptr(), DTYPE_BF16, x.shape[0],
+                                      y.data_ptr(), DTYPE_BF16, _stream(self.raw.device)))
+        return y
+
     def linear(self, x: torch.Tensor) -> torch.Tensor:
         self.to_gpu()
         flat = x.reshape(-1, x.shape[-1]).to(self.device)
         if flat.shape[0] <= MAX_TOKENS:
-            y = gemv(self.raw, self.type_name, self.shape, flat).to(x.dtype)
+            if x.dtype == torch.bfloat16:
+                y = self._gemv_bf16(flat)
+            else:
+                y = gemv(self.raw, self.type_name, self.shape, flat).to(x.dtype)
         elif self.keep_dense:  # the reference's arithmetic (gguf/metal.py:407) on bf16 values kept in HBM
             y = F.linear(flat.to(torch.bfloat16), self.dense()).to(x.dtype)
         else:  # the reference's own form (gguf/metal.py:407): dequantized on every call, nothing kept
