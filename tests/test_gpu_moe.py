@@ -346,6 +346,19 @@ def test_prefill_mfma_variants(hip, variant):
     check_prefill(hip, layer, lw, synth.tokens(71, T, kw["hidden"]), variant)
 
 
+@pytest.mark.parametrize("gate_up,down,inter,T", [
+    ("Q4_K", "Q6_K", 512, 80), ("Q4_K", "Q6_K", 512, 81), ("Q4_K", "Q4_K", 256, 97), ("Q6_K", "Q6_K", 1024, 112),
+    ("Q6_K", "Q4_K", 512, 113), ("Q4_K", "Q6_K", 1024, 129), ("Q6_K", "Q6_K", 256, 256)])
+def test_prefill_small_tiles(hip, gate_up, down, inter, T):
+    """The 64-token-tile GEMMs (at most 64 tokens per expert on average): the shared expert's last tile holds 16, 17,
+    33, 48, 49, 1 and 64 tokens (each count of 16-token tiles, full and just begun), the routed ones what the routing
+    gives; one to four blocks per down row (activations resident or staged in phases), both types each way. The bound
+    is the other MFMA tests' (bf16 roundings falling the other way)."""
+    lw = synth.moe_layer(72, hidden=1024, inter=inter, shared_inter=inter, experts=16, top_k=4, gate_up_type=gate_up,
+                         down_type=down)
+    check_prefill(hip, hip.MoELayer.from_host(lw, mfma="always"), lw, synth.tokens(73, T, 1024), f"small tiles {T}")
+
+
 @pytest.mark.parametrize("T", [12, 64])
 def test_mfma_small_batches_k_split(hip, layer_c2, T):
     """At most 64 tokens with every expert on the MFMA GEMMs (the full-shape layer): the K-split kernels, gate_up's

@@ -70,6 +70,14 @@ __device__ __forceinline__ const uint32_t* align_down4(const uint8_t* p, uint32_
     return reinterpret_cast<const uint32_t*>(p - sh);
 }
 
+// A value from a 2-byte-aligned address in one load (global loads take any alignment on amdhsa).
+template <typename V>
+__device__ __forceinline__ V load_a2(const uint8_t* p) {
+    V v;
+    __builtin_memcpy(&v, __builtin_assume_aligned(p, 2), sizeof(V));
+    return v;
+}
+
 __device__ __forceinline__ uint4 load16_a2(const uint8_t* p) {
     uint32_t sh;
     const uint32_t* q = align_down4(p, sh);

@@ -72,6 +72,7 @@ struct ExpertArgs {
 constexpr int kTileTokens = 144;             // prefill: tokens per gate_up GEMM tile (9 MFMA token tiles)
 constexpr int kDownTileTokens = 128;         // prefill: tokens per down GEMM tile (8 MFMA token tiles)
 constexpr int kDownSlabsMax = 4;            // prefill: most 256-row slabs per down workgroup
+constexpr int kSmallTileTokens = 64;         // prefill with few tokens per expert: tokens per tile of both GEMMs
 // An expert given at most this many tokens runs on the fp32 GEMV kernels with exact weights, one given more on the
 // bf16 MFMA GEMMs: the reference applies the rule of gguf/metal.py:20,404-407 to each expert's own tokens
 // (engines/base.py:566-571).
@@ -91,7 +92,7 @@ struct PrefillArgs {
     const int32_t* sorted;   // [T*k] pair id by sorted position
     const int4* tiles;       // gate_up tiles: (expert or E for the shared expert, first position / token, count)
     const int32_t* n_tiles;
-    const int4* tiles_down;  // down tiles, the same of at most kDownTileTokens tokens
+    const int4* tiles_down;  // down tiles, for the down GEMM's tile size
     const int32_t* n_tiles_down;
     uint16_t* h16;           // [T*k, inter] bf16 by sorted position
     uint16_t* h_sh16;        // [T, shared_inter] bf16
@@ -124,8 +125,8 @@ struct Workspace {
     float* o_sh;        // [T, hidden]
     // prefill (MFMA) path only
     uint16_t* xb;       // [T, hidden] bf16
-    int4* tiles;        // [max_tiles(kTileTokens)]
-    int4* tiles_down;   // [max_tiles(kDownTileTokens)]
+    int4* tiles;        // [max_tiles(tile_caps().gate_up)]
+    int4* tiles_down;   // [max_tiles(tile_caps().down)]
     int32_t* n_tiles;   // [2]: gate_up tiles, down tiles
     uint16_t* h16;      // [T*k, inter] bf16
     uint16_t* h_sh16;   // [T, shared_inter] bf16
@@ -153,6 +154,11 @@ inline int plan_gemv_max(ExpertPlan plan) {
     return plan == kPlanMfma ? 0 : plan == kPlanSplit ? kGemvMaxTokens : 0x7FFFFFFF;
 }
 int max_tiles(const WlMoeLayer& L, int64_t T, int cap, int gemv_max);
+// Tokens per tile of a call's two GEMM tile lists.
+struct TileCaps {
+    int gate_up, down;
+};
+TileCaps tile_caps(const WlMoeLayer& L, int64_t T);
 int launch_router_tiled(const WlMoeLayer& L, const float* x, int64_t T, float* logits, float* sg, uint16_t* xb,
                         hipStream_t s);
 // with_gemv: the call also has GEMV experts (a split plan), which may run beside this launch on a second stream;

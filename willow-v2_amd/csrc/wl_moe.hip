@@ -368,10 +368,11 @@ __device__ __forceinline__ int chunk_rank(const uint32_t* bits, int e, int t) {
 // experts), and the table entries of MFMA experts' pairs carry kPosBf16.
 struct TileOut {
     int4* tiles;
-    int4* tiles_down;
+    int4* tiles_down;  // the same list as tiles when the tile sizes are equal
     int32_t* n_tiles;
     int with_shared;
     int gemv_max;
+    TileCaps caps;  // tokens per tile of each list
 };
 
 __global__ __launch_bounds__(1024) void k_sort_hist(const int32_t* __restrict__ ids, int T, int k, int E,
@@ -562,7 +563,7 @@ __device__ __forceinline__ void sort_small(const int32_t* __restrict__ ids, int 
     if (e < E)
 #pragma unroll
         for (int wd = 0; wd < kSortWords; wd++) c += __popc(bits[kSortWords * e + wd]);
-    if (P <= 1024 && E <= 256 && T <= kDownTileTokens) {
+    if (P <= 1024 && E <= 256 && T <= min(to.caps.gate_up, to.caps.down)) {
         // Few pairs (batched decode): every MFMA expert and the shared expert fit one tile of either list, so
         // the four scans below (positions, GEMV experts, the two tile lists) are one scan of three packed counts:
         // pairs in bits 0..10 (<= 1024), GEMV experts in 11..19 and MFMA experts in 20..28 (<= 256 each), whose
@@ -637,8 +638,9 @@ __device__ __forceinline__ void sort_small(const int32_t* __restrict__ ids, int 
             po.put(q, k, entry, po.crank[q], po.wts[q]);
     }
     if (to.tiles) {
-        tile_list(to.tiles, to.n_tiles, kTileTokens, e, E, big ? c : 0, off, T, to.with_shared, wsum);
-        tile_list(to.tiles_down, to.n_tiles + 1, kDownTileTokens, e, E, big ? c : 0, off, T, to.with_shared, wsum);
+        tile_list(to.tiles, to.n_tiles, to.caps.gate_up, e, E, big ? c : 0, off, T, to.with_shared, wsum);
+        if (to.tiles_down != to.tiles)
+            tile_list(to.tiles_down, to.n_tiles + 1, to.caps.down, e, E, big ? c : 0, off, T, to.with_shared, wsum);
     }
     if (fork_sync) publish_grouping(fork_sync, withhold);
 }
@@ -745,8 +747,9 @@ __global__ __launch_bounds__(kSortSmallThreads) void k_sort_scan(int T, int k, i
     if (mine && c > 0 && !big) active[1 + apos] = e;
     if (threadIdx.x == 0) active[0] = total;
     if (to.tiles) {
-        tile_list(to.tiles, to.n_tiles, kTileTokens, e, E, big ? c : 0, off, T, to.with_shared, wsum);
-        tile_list(to.tiles_down, to.n_tiles + 1, kDownTileTokens, e, E, big ? c : 0, off, T, to.with_shared, wsum);
+        tile_list(to.tiles, to.n_tiles, to.caps.gate_up, e, E, big ? c : 0, off, T, to.with_shared, wsum);
+        if (to.tiles_down != to.tiles)
+            tile_list(to.tiles_down, to.n_tiles + 1, to.caps.down, e, E, big ? c : 0, off, T, to.with_shared, wsum);
     }
 }
 
@@ -1338,9 +1341,13 @@ Workspace carve(const WlMoeLayer& L, int64_t T, void* base) {
     const ExpertPlan plan = expert_plan(L, T);
     const bool mfma = plan != kPlanGemv;
     const int gmax = plan_gemv_max(plan);
+    const TileCaps caps = tile_caps(L, T);
     w.xb = static_cast<uint16_t*>(take(mfma ? sizeof(uint16_t) * T * L.hidden : 0));
-    w.tiles = static_cast<int4*>(take(mfma ? sizeof(int4) * max_tiles(L, T, kTileTokens, gmax) : 0));
-    w.tiles_down = static_cast<int4*>(take(mfma ? sizeof(int4) * max_tiles(L, T, kDownTileTokens, gmax) : 0));
+    w.tiles = static_cast<int4*>(take(mfma ? sizeof(int4) * max_tiles(L, T, caps.gate_up, gmax) : 0));
+    // with equal tile sizes the two lists are one (so the smaller tiles never need more workspace)
+    w.tiles_down = caps.down == caps.gate_up
+                       ? w.tiles
+                       : static_cast<int4*>(take(mfma ? sizeof(int4) * max_tiles(L, T, caps.down, gmax) : 0));
     w.n_tiles = static_cast<int32_t*>(take(mfma ? 2 * sizeof(int32_t) : 0));
     w.h16 = static_cast<uint16_t*>(take(mfma ? sizeof(uint16_t) * P * L.inter : 0));
     w.h_sh16 = static_cast<uint16_t*>(take(mfma && shared ? sizeof(uint16_t) * T * L.shared_inter : 0));
@@ -1473,7 +1480,7 @@ static int launch_topk_parts(const WlMoeLayer& L, int64_t T, const Workspace& w,
 static int launch_sort(const WlMoeLayer& L, const Workspace& w, const int32_t* ids, int64_t T, bool tiles,
                        int gemv_max, bool fork, bool withhold, hipStream_t s) {
     const int E = L.n_experts, k = L.top_k;
-    const TileOut to{tiles ? w.tiles : nullptr, w.tiles_down, w.n_tiles, L.shared_gate_up ? 1 : 0, gemv_max};
+    const TileOut to{tiles ? w.tiles : nullptr, w.tiles_down, w.n_tiles, L.shared_gate_up ? 1 : 0, gemv_max, tile_caps(L, T)};
     const int nchunks = static_cast<int>((T + kSortChunk - 1) / kSortChunk);
     if (nchunks == 1) {
         k_sort_small<<<1, kSortSmallThreads, 0, s>>>(ids, static_cast<int>(T), k, E, w.offsets, w.active, w.sorted,
@@ -1794,7 +1801,8 @@ static int run_layer(const WlMoeLayer* layer, const float* x, int64_t tokens, fl
         mark(1);
         // the grouping in the same launch (mark 3 follows mark 2 at once)
         const GroupOut g{w.offsets, w.active, w.sorted, PickOut{w.crank, w.wts, w.picks},
-                         TileOut{mfma ? w.tiles : nullptr, w.tiles_down, w.n_tiles, L.shared_gate_up ? 1 : 0, gemv_max},
+                         TileOut{mfma ? w.tiles : nullptr, w.tiles_down, w.n_tiles, L.shared_gate_up ? 1 : 0, gemv_max,
+                                 tile_caps(L, tokens)},
                          w.sync, in_scope ? 1 : 0, starve ? 1 : 0};
         rc = launch_topk_parts(L, tokens, w, sg, &g, s);
         if (rc) return rc;

@@ -36,15 +36,15 @@ constexpr int tile_bytes() { return TILE * kTileRowBytes; }  // one LDS buffer: 
 constexpr int kRT = 2;
 constexpr int kGemmWaves = 16 / kRT;
 constexpr int kGemmThreads = 64 * kGemmWaves;
-
-// 8 bytes from a 2-byte-aligned address: 3 aligned dwords, realigned. Reads [p & ~3, (p & ~3) + 12), within
-// [p - 2, p + 12); all three loads are unconditional so that no branch splits the wavefront.
-__device__ __forceinline__ uint2 load8_a2(const uint8_t* p) {
-    uint32_t sh;
-    const uint32_t* q = align_down4(p, sh);
-    const uint32_t w0 = q[0], w1 = q[1], w2 = q[2];
-    return make_uint2(__builtin_amdgcn_alignbyte(w1, w0, sh), __builtin_amdgcn_alignbyte(w2, w1, sh));
-}
+// Small tiles (kSmallTileTokens): workgroups of 4 wavefronts and 8 row tiles, three on a CU.
+constexpr int kSmallWaves = 4;
+constexpr int kSmallLds = 48 << 10;
+template <int TILE>
+constexpr int gemm_wg_waves() { return TILE == kSmallTileTokens ? kSmallWaves : kGemmWaves; }
+template <int TILE>
+constexpr int gemm_rows() { return 16 * kRT * gemm_wg_waves<TILE>(); }  // weight rows of a workgroup
+template <int TILE>
+constexpr int gemm_lds() { return TILE == kSmallTileTokens ? kSmallLds : 2 * tile_bytes<TILE>(); }
 
 // ---------------------------------------------------------------------------------------------------------------
 // Router for many tokens on the matrix core. v_mfma_f32_16x16x4_f32 computes each output as four fused multiply-adds
@@ -287,8 +287,21 @@ struct Q6KRowState {
     float a[4];    // value = a[t] * (q6 - 32), a[t] = d * scale 8 h + 2 t + p
 };
 
+// WIDE: each field in one load from its 2-byte-aligned address (5 loads and 15 registers in flight) instead of aligned
+// dwords realigned in registers (19 loads). The memory system splits the wide loads that cross a 64-byte line, so they
+// pay where registers and issue bind (small tiles: 1000 tokens, down 108 -> 93 us) and cost where the loads are hidden
+// under many MFMAs anyway (128-token tiles: 170 -> 187 us at 2800 tokens).
+template <bool WIDE>
 __device__ __forceinline__ void fetch_q6k(const uint8_t* __restrict__ blk, int q, Q6KRowState& s) {
     const int h = q >> 1, p = q & 1;
+    if constexpr (WIDE) {
+        s.ql[0] = load_a2<uint4>(blk + 64 * h + 16 * p);
+        s.ql[1] = load_a2<uint4>(blk + 64 * h + 32 + 16 * p);
+        s.qh = load_a2<uint4>(blk + 128 + 32 * h + 16 * p);
+        s.sc = load_a2<uint2>(blk + 192 + 8 * h);
+        s.d = half_to_float(*reinterpret_cast<const uint16_t*>(blk + 208));
+        return;
+    }
     s.ql[0] = load16_a2(blk + 64 * h + 16 * p);
     s.ql[1] = load16_a2(blk + 64 * h + 32 + 16 * p);
     s.qh = load16_a2(blk + 128 + 32 * h + 16 * p);
@@ -337,20 +350,20 @@ __device__ __forceinline__ bf16x8 fragment_q6k(const Q6KRowState& s) {
     return __builtin_bit_cast(bf16x8, p);
 }
 
-template <int TYPE>
+template <int TYPE, bool WIDE = false>
 struct RowState;
-template <>
-struct RowState<WL_TYPE_Q4_K> {
+template <bool WIDE>
+struct RowState<WL_TYPE_Q4_K, WIDE> {
     Q4KRowState s;
     __device__ __forceinline__ void fetch(const uint8_t* blk, int q) { fetch_q4k(blk, q, s); }
     __device__ __forceinline__ void prepare(int q) { prepare_q4k(s, q); }
     template <int KK>
     __device__ __forceinline__ bf16x8 frag(int) const { return fragment_q4k<KK>(s); }
 };
-template <>
-struct RowState<WL_TYPE_Q6_K> {
+template <bool WIDE>
+struct RowState<WL_TYPE_Q6_K, WIDE> {
     Q6KRowState s;
-    __device__ __forceinline__ void fetch(const uint8_t* blk, int q) { fetch_q6k(blk, q, s); }
+    __device__ __forceinline__ void fetch(const uint8_t* blk, int q) { fetch_q6k<WIDE>(blk, q, s); }
     __device__ __forceinline__ void prepare(int q) { prepare_q6k(s, q); }
     template <int KK>
     __device__ __forceinline__ bf16x8 frag(int) const { return fragment_q6k<KK>(s); }
@@ -420,8 +433,8 @@ constexpr bool kSchedGroups = false;
 // fragments are decoded at the top of the next iteration) and, as each b[n] has been consumed, reading step
 // KK + 1's b[n] in its place (the last step's successor reads from the other LDS buffer after the barrier), so the
 // decode runs while the matrix core is busy.
-template <int TYPE, int NT, int KK, int NTA>
-__device__ __forceinline__ void gemm_step(const uint8_t* buf, const BAddr& ba, const RowState<TYPE> (&rs)[kRT],
+template <int TYPE, int NT, int KK, int NTA, bool WIDE>
+__device__ __forceinline__ void gemm_step(const uint8_t* buf, const BAddr& ba, const RowState<TYPE, WIDE> (&rs)[kRT],
                                           floatx4 (&acc)[kRT][NTA], const bf16x8 (&a)[kRT], bf16x8 (&b)[NT],
                                           bf16x8 (&an)[kRT], int q) {
 #pragma unroll
@@ -457,36 +470,38 @@ __device__ __forceinline__ void gemm_step(const uint8_t* buf, const BAddr& ba, c
 // The loads are issued from inline assembly so that the compiler, which cannot tell the two LDS buffers apart,
 // does not wait for them before the next LDS read of the other buffer; the K loop waits for them itself
 // (s_waitcnt vmcnt(0) and a barrier) before the buffer is read.
-template <int TILE>
-constexpr int stage_iters() { return tile_bytes<TILE>() / (kGemmWaves * 1024); }  // 9 for 144 tokens
+template <int TILE, int W = kGemmWaves>
+constexpr int stage_iters() { return TILE / (2 * W); }  // 9 for 144 tokens
 static_assert(kGemmWaves % 8 == 0 && kTileTokens % (2 * kGemmWaves) == 0 && kDownTileTokens % (2 * kGemmWaves) == 0,
               "");
-template <int TILE>
+template <int TILE, int W = kGemmWaves>
 __host__ __device__ constexpr int rowtab_index(int t) {
-    return stage_iters<TILE>() * (t % (2 * kGemmWaves)) + t / (2 * kGemmWaves);
+    return stage_iters<TILE, W>() * (t % (2 * W)) + t / (2 * W);
 }
 
 __device__ __forceinline__ uint32_t lds_address(const void* p) {
     return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void*)(p)));
 }
 
-template <int TILE, int NT>
+// With W = 4 (small tiles) the 8 rows of odd instructions sit 8 rows on, which a swizzle of 15 (col8 = 128: bit 3 of
+// the slot) tells apart.
+template <int TILE, int NT, int W = kGemmWaves>
 __device__ __forceinline__ void stage_async(uint32_t buf, const uint8_t* src, const uint32_t* rowtab, uint32_t col,
-                                            int wv, int half) {
-    constexpr int kIters = stage_iters<TILE>();
-    static_assert(NT <= kIters, "");
+                                            int wv, int half, uint32_t col8 = 0) {
+    constexpr int kIters = stage_iters<TILE, W>(), kUsed = 8 * NT / W;
+    static_assert(kUsed <= kIters && (W == 8 || W == 4), "");
     const uint32_t* tab = rowtab + kIters * (2 * wv + half);
-    uint32_t off[NT];
+    uint32_t off[kUsed];
 #pragma unroll
-    for (int i = 0; i < NT; i++) off[i] = tab[i];
+    for (int i = 0; i < kUsed; i++) off[i] = tab[i];
 #pragma unroll
-    for (int it = 0; it < NT; it++) {  // iteration it: tokens 16 it .. 16 it + 15, token tile it
+    for (int it = 0; it < kUsed; it++) {  // iteration it: tokens 2 W it .. 2 W it + 2 W - 1
         // M0 (the LDS destination) is a register the compiler reserves: saved and restored around the load
         uint32_t saved;
         asm volatile(
             "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3\n\ts_mov_b32 m0, %0"
             : "=&s"(saved)
-            : "s"(buf + (kGemmWaves * it + wv) * 1024), "v"(off[it] + col), "s"(src)
+            : "s"(buf + (W * it + wv) * 1024), "v"(off[it] + (W == 4 && (it & 1) ? col ^ col8 : col)), "s"(src)
             : "memory");
     }
 }
@@ -670,37 +685,126 @@ __device__ __forceinline__ void gemm_loop_small(uint8_t (&bufs)[2][tile_bytes<TI
     }
 }
 
+// The K loop of the small-tile kernels (experts of a few dozen tokens), which stream the weights: what bounds it is
+// neither the decode nor the matrix core (without the decode's arithmetic 110 -> 105 us at 1000 tokens' gate_up) but
+// the round trips of a workgroup's short chain. So workgroups are half as many wavefronts with a third of a CU's LDS,
+// three on a CU, at 168 registers, and the token tiles are exact (NT = 1 .. 4, not 1 or 4); a wavefront requests its
+// next row states at each step, and the activation chunks are staged as many at a time as the LDS holds (once for
+// all items when every chunk fits). One workgroup of 8 wavefronts per CU before: 1000 tokens, gate_up 158 -> 110 us,
+// down 137 -> 93. Measured and not taken: the chunks double-buffered with a barrier per block (gate_up 116), four
+// workgroups of 36 KiB (128 registers, layer 294 -> 314), two of 72 KiB with twice the slots (323), an L2 prefetch of
+// the next phase's lines (314). Same results as gemm_loop: the same fragments and MFMAs in the same order.
+template <int TYPE, int NT, int NTA, typename RowPtr, typename Epilogue>
+__device__ __forceinline__ void gemm_loop_tiny(uint8_t* lds, floatx4 (&acc)[kRT][NTA], int nblocks, int nitems,
+                                              const uint8_t* src, const uint32_t* rowtab, RowPtr row_ptr, Epilogue epi,
+                                              int lr, int q) {
+    constexpr int kChunk = NT * 16 * kTileRowBytes;
+    constexpr int kSlots = kSmallLds / kChunk;
+    static_assert(NT <= NTA && kSlots >= 1, "");
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)), half = lane >> 5;
+    const uint32_t col = 16u * static_cast<uint32_t>((lane & 31) ^ ((2 * wv + half) & swizzle<TYPE>()));
+    const uint32_t lds0 = lds_address(lds);
+    const BAddr ba = b_addr<TYPE>(lr, q);
+    const bool resident = nblocks <= kSlots;
+    RowState<TYPE, true> rs[kRT], nx[kRT];
+#pragma unroll
+    for (int r = 0; r < kRT; r++) rs[r].fetch(row_ptr(0, r, lr), q);
+    bf16x8 a0[kRT], a1[kRT], b[NT];
+    int item = 0, kc = 0, slot = 0;
+    for (;;) {
+        if (resident ? (item == 0 && kc == 0) : slot == 0) {
+            __syncthreads();  // every wavefront is done with the chunks that are replaced
+            const int n = resident ? nblocks : min(kSlots, nblocks - kc);
+            for (int c = 0; c < n; c++)
+                stage_async<kSmallTileTokens, NT, kSmallWaves>(lds0 + c * kChunk,
+                                                               src + static_cast<int64_t>(kc + c) * kTileRowBytes,
+                                                               rowtab, col, wv, half, TYPE == WL_TYPE_Q4_K ? 0u : 128u);
+            wait_stage();
+            __syncthreads();
+        }
+        const bool item_end = kc == nblocks - 1;
+        const bool last = item_end && item == nitems - 1;
+        const int in = item_end && !last ? item + 1 : item, kn = item_end ? 0 : kc + 1;
+        const uint8_t* buf = lds + slot * kChunk;
+        read_b<TYPE, NT, 0>(buf, ba, b);
+#pragma unroll
+        for (int r = 0; r < kRT; r++)
+            nx[r].fetch(row_ptr(in, r, lr) + static_cast<int64_t>(kn) * BlockInfo<TYPE>::bytes, q);
+#pragma unroll
+        for (int r = 0; r < kRT; r++) {
+            rs[r].prepare(q);
+            a0[r] = rs[r].template frag<0>(q);
+        }
+        gemm_step<TYPE, NT, 0, NTA>(buf, ba, rs, acc, a0, b, a1, q);
+        gemm_step<TYPE, NT, 1, NTA>(buf, ba, rs, acc, a1, b, a0, q);
+        gemm_step<TYPE, NT, 2, NTA>(buf, ba, rs, acc, a0, b, a1, q);
+        gemm_step<TYPE, NT, 3, NTA>(buf, ba, rs, acc, a1, b, a0, q);
+        gemm_step<TYPE, NT, 4, NTA>(buf, ba, rs, acc, a0, b, a1, q);
+        gemm_step<TYPE, NT, 5, NTA>(buf, ba, rs, acc, a1, b, a0, q);
+        gemm_step<TYPE, NT, 6, NTA>(buf, ba, rs, acc, a0, b, a1, q);
+        gemm_step<TYPE, NT, 7, NTA>(buf, ba, rs, acc, a1, b, a0, q);
+#pragma unroll
+        for (int r = 0; r < kRT; r++) rs[r] = nx[r];
+        if (item_end) {
+            epi(item, acc);
+#pragma unroll
+            for (int r = 0; r < kRT; r++)
+#pragma unroll
+                for (int n = 0; n < NTA; n++) acc[r][n] = floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+        if (last) break;
+        item = in;
+        kc = kn;
+        slot = resident ? kc : (item_end || slot == kSlots - 1 ? 0 : slot + 1);
+    }
+}
+
 // ---------------------------------------------------------------------------------------------------------------
 // The GEMM core: a workgroup of kGemmWaves wavefronts, each owning kRT row tiles of 16 (rows given by
 // row_ptr(item, r, lr), for nitems row sets one after another) and the tile's up to TILE tokens as NT token tiles of
 // 16 (NT = TILE / 16, 8, 4 or 1, the fewest that cover `count`; only those are staged). Per K chunk of 256 values
 // (one block per row) the activations sit in LDS (double-buffered in gemm_loop; staged a phase at a time in
-// gemm_loop_small, which takes NT = 4 and 1), and each of the 8 32-value steps decodes kRT A-fragments and runs
-// kRT x NT MFMAs; epi(item, acc) stores each row set's results. src_row(t) is token t's row in src ([*, ld] bf16);
-// rows past count load token 0's (their results are never stored).
+// gemm_loop_small, which takes NT = 4 and 1, and gemm_loop_tiny, which runs every tile of a small-tile kernel), and
+// each of the 8 32-value steps decodes kRT A-fragments and runs kRT x NT MFMAs; epi(item, acc) stores each row set's
+// results. src_row(t) is token t's row in src ([*, ld] bf16); rows past count load token 0's (their results are never
+// stored).
 template <int TYPE, int TILE, typename RowPtr, typename SrcRow, typename Epilogue>
-__device__ __forceinline__ void gemm_tile(uint8_t (&bufs)[2][tile_bytes<TILE>()], floatx4 (&acc)[kRT][TILE / 16],
+__device__ __forceinline__ void gemm_tile(uint8_t (&bufs)[gemm_lds<TILE>()], floatx4 (&acc)[kRT][TILE / 16],
                                           int nblocks, int nitems, int count, const uint16_t* __restrict__ src,
                                           int64_t ld, SrcRow src_row, RowPtr row_ptr, Epilogue epi) {
     constexpr int NTA = TILE / 16;
     __shared__ __attribute__((aligned(16))) uint32_t rowtab[TILE];
     const int lane = threadIdx.x & 63, lr = lane & 15, q = lane >> 4;
     for (int t = threadIdx.x; t < TILE; t += blockDim.x)
-        rowtab[rowtab_index<TILE>(t)] = static_cast<uint32_t>(src_row(t < count ? t : 0) * ld * 2);
+        rowtab[rowtab_index<TILE, gemm_wg_waves<TILE>()>(t)] =
+            static_cast<uint32_t>(src_row(t < count ? t : 0) * ld * 2);
 #pragma unroll
     for (int r = 0; r < kRT; r++)
 #pragma unroll
         for (int n = 0; n < NTA; n++) acc[r][n] = floatx4{0.f, 0.f, 0.f, 0.f};
     __syncthreads();
     const uint8_t* s8 = uniform_ptr(reinterpret_cast<const uint8_t*>(src));
-    if (NTA > 8 && count > 128)
-        gemm_loop<TYPE, TILE, NTA, NTA>(bufs, acc, nblocks, nitems, s8, rowtab, row_ptr, epi, lr, q);
-    else if (count > 64)
-        gemm_loop<TYPE, TILE, 8, NTA>(bufs, acc, nblocks, nitems, s8, rowtab, row_ptr, epi, lr, q);
-    else if (count > 16)
-        gemm_loop_small<TYPE, TILE, 4, NTA>(bufs, acc, nblocks, nitems, s8, rowtab, row_ptr, epi, lr, q);
-    else
-        gemm_loop_small<TYPE, TILE, 1, NTA>(bufs, acc, nblocks, nitems, s8, rowtab, row_ptr, epi, lr, q);
+    if constexpr (TILE == kSmallTileTokens) {
+        if (count > 48)
+            gemm_loop_tiny<TYPE, 4, NTA>(bufs, acc, nblocks, nitems, s8, rowtab, row_ptr, epi, lr, q);
+        else if (count > 32)
+            gemm_loop_tiny<TYPE, 3, NTA>(bufs, acc, nblocks, nitems, s8, rowtab, row_ptr, epi, lr, q);
+        else if (count > 16)
+            gemm_loop_tiny<TYPE, 2, NTA>(bufs, acc, nblocks, nitems, s8, rowtab, row_ptr, epi, lr, q);
+        else
+            gemm_loop_tiny<TYPE, 1, NTA>(bufs, acc, nblocks, nitems, s8, rowtab, row_ptr, epi, lr, q);
+    } else {
+        auto& two = reinterpret_cast<uint8_t (&)[2][tile_bytes<TILE>()]>(bufs);
+        if (NTA > 8 && count > 128)
+            gemm_loop<TYPE, TILE, NTA, NTA>(two, acc, nblocks, nitems, s8, rowtab, row_ptr, epi, lr, q);
+        else if (count > 64)
+            gemm_loop<TYPE, TILE, 8, NTA>(two, acc, nblocks, nitems, s8, rowtab, row_ptr, epi, lr, q);
+        else if (count > 16)
+            gemm_loop_small<TYPE, TILE, 4, NTA>(two, acc, nblocks, nitems, s8, rowtab, row_ptr, epi, lr, q);
+        else
+            gemm_loop_small<TYPE, TILE, 1, NTA>(two, acc, nblocks, nitems, s8, rowtab, row_ptr, epi, lr, q);
+    }
 }
 
 // Workgroups are dealt to the 8 XCDs round-robin by linear id, each XCD with its own L2. slab_tile maps the linear
@@ -716,22 +820,23 @@ __device__ __forceinline__ void slab_tile(int nslab, int& slab, int& tile) {
 
 // gate_up: slab = 128-row slab of the intermediate dim; wavefront w: gate rows j0 + 16r + lr (r < kRT / 2)
 // and the matching up rows inter + j0 + ... (r >= kRT / 2), j0 = 128 slab + 8 kRT w. Epilogue h = silu(g) * u -> bf16.
-// TILE is kTileTokens, or kDownTileTokens (and the down tile list) for Q6_K rows, whose larger row state leaves no
-// registers for a ninth token tile.
+// TILE is tile_caps().gate_up: kTileTokens, kDownTileTokens for Q6_K rows (whose larger row state leaves no registers
+// for a ninth token tile), or kSmallTileTokens, whose slabs are 64 rows.
 template <int TYPE, int TILE>
-__global__ __launch_bounds__(kGemmThreads) void k_gemm_gate_up(PrefillArgs a) {
-    __shared__ __attribute__((aligned(16))) uint8_t bufs[2][tile_bytes<TILE>()];
+__global__ __launch_bounds__(64 * gemm_wg_waves<TILE>(), TILE == kSmallTileTokens ? 3 : 2)
+    void k_gemm_gate_up(PrefillArgs a) {
+    __shared__ __attribute__((aligned(16))) uint8_t bufs[gemm_lds<TILE>()];
     if (a.skip && *a.skip) return;
     int slab, ti;
     slab_tile(a.nslab_gate_up, slab, ti);
-    const int4* tiles = TILE == kTileTokens ? a.tiles : a.tiles_down;
-    if (ti >= (TILE == kTileTokens ? a.n_tiles[0] : a.n_tiles_down[0])) return;
-    const int4 tile = tiles[ti];
+    if (ti >= a.n_tiles[0]) return;
+    const int4 tile = a.tiles[ti];
     const bool sh = tile.x == a.E;
     const int inter = sh ? a.sh_inter : a.inter;
     constexpr int kHalf = kRT / 2;
-    const int j0 = slab * 128 + 16 * kHalf * (threadIdx.x >> 6);
-    if (slab * 128 >= inter) return;
+    constexpr int kSlab = gemm_rows<TILE>() / 2;
+    const int j0 = slab * kSlab + 16 * kHalf * (threadIdx.x >> 6);
+    if (slab * kSlab >= inter) return;
     const uint8_t* W = sh ? a.sh_gate_up : a.gate_up + static_cast<int64_t>(tile.x) * a.gate_up_stride;
     const int nb = a.H / kQK;
     const int64_t rs = static_cast<int64_t>(nb) * BlockInfo<TYPE>::bytes;
@@ -762,56 +867,58 @@ __global__ __launch_bounds__(kGemmThreads) void k_gemm_gate_up(PrefillArgs a) {
     gemm_tile<TYPE, TILE>(bufs, acc, nb, 1, count, a.xb, a.H, src_row, row_ptr, epi);
 }
 
-// down: a workgroup takes a.down_slabs consecutive 256-row slabs of the hidden dim (one pipeline across them); for
+// down: a workgroup takes a.down_slabs consecutive 256-row slabs (128 with small tiles) of the hidden dim (one pipeline across them); for
 // slab item, wavefront w has rows 256 (slab0 + item) + 16 kRT w + 16 r + lr. o by position (row stride a.ldo;
 // the shared expert's by token, stride H), rounded to bf16 as the reference's bf16 F.linear output is
 // (gguf/metal.py:407). Its tiles hold at most 128 tokens (8 token tiles of accumulators keep Q6_K's wavefronts
 // within 256 registers).
-template <int TYPE>
-__global__ __launch_bounds__(kGemmThreads) void k_gemm_down(PrefillArgs a) {
-    __shared__ __attribute__((aligned(16))) uint8_t bufs[2][tile_bytes<kDownTileTokens>()];
+template <int TYPE, int TILE>
+__global__ __launch_bounds__(64 * gemm_wg_waves<TILE>(), TILE == kSmallTileTokens ? 3 : 2)
+    void k_gemm_down(PrefillArgs a) {
+    __shared__ __attribute__((aligned(16))) uint8_t bufs[gemm_lds<TILE>()];
     if (a.skip && *a.skip) return;
     int group, ti;
-    slab_tile(a.H / 256 / a.down_slabs, group, ti);
+    constexpr int kRows = gemm_rows<TILE>();
+    slab_tile(a.H / kRows / a.down_slabs, group, ti);
     int4 tile;
     if (a.dense_tokens > 0) {  // wl_linear: token tile ti of one matrix
-        const int p = ti * kDownTileTokens;
+        const int p = ti * TILE;
         if (p >= a.dense_tokens) return;
-        tile = make_int4(0, p, min(kDownTileTokens, a.dense_tokens - p), 0);
+        tile = make_int4(0, p, min(TILE, a.dense_tokens - p), 0);
     } else {
         if (ti >= a.n_tiles_down[0]) return;
         tile = a.tiles_down[ti];
     }
     const bool sh = tile.x == a.E;
     const int inter = sh ? a.sh_inter : a.inter;
-    const int row0 = group * a.down_slabs * 256 + 16 * kRT * (threadIdx.x >> 6);
+    const int row0 = group * a.down_slabs * kRows + 16 * kRT * (threadIdx.x >> 6);
     const uint8_t* W = sh ? a.sh_down : a.down + static_cast<int64_t>(tile.x) * a.down_stride;
     const int nb = inter / kQK;
     const int64_t rs = static_cast<int64_t>(nb) * BlockInfo<TYPE>::bytes;
     const int pos0 = tile.y, count = tile.z;
-    floatx4 acc[kRT][kDownTileTokens / 16];
+    floatx4 acc[kRT][TILE / 16];
     auto row_ptr = [&](int item, int r, int lr) {
-        return W + static_cast<int64_t>(row0 + 256 * item + 16 * r + lr) * rs;
+        return W + static_cast<int64_t>(row0 + kRows * item + 16 * r + lr) * rs;
     };
     auto src_row = [&](int t) -> int64_t { return pos0 + t; };
     uint16_t* out = sh ? a.o_sh16 : a.o16;
     const int64_t ldo = sh ? a.H : a.ldo;
-    auto epi = [&](int item, floatx4 (&acc)[kRT][kDownTileTokens / 16]) {
+    auto epi = [&](int item, floatx4 (&acc)[kRT][TILE / 16]) {
         const int lane = threadIdx.x & 63, lr = lane & 15, q = lane >> 4;
 #pragma unroll
         for (int r = 0; r < kRT; r++) {
 #pragma unroll
-            for (int n = 0; n < kDownTileTokens / 16; n++) {
+            for (int n = 0; n < TILE / 16; n++) {
                 const int t = 16 * n + lr;
                 if (t < count) {
                     const floatx4 v = acc[r][n];
-                    *reinterpret_cast<uint2*>(out + static_cast<int64_t>(pos0 + t) * ldo + row0 + 256 * item +
+                    *reinterpret_cast<uint2*>(out + static_cast<int64_t>(pos0 + t) * ldo + row0 + kRows * item +
                                               16 * r + 4 * q) = make_uint2(pack2(v[0], v[1]), pack2(v[2], v[3]));
                 }
             }
         }
     };
-    gemm_tile<TYPE, kDownTileTokens>(bufs, acc, nb, a.down_slabs, count, sh ? a.h_sh16 : a.h16, inter, src_row,
+    gemm_tile<TYPE, TILE>(bufs, acc, nb, a.down_slabs, count, sh ? a.h_sh16 : a.h16, inter, src_row,
                                      row_ptr, epi);
 }
 
@@ -1033,6 +1140,10 @@ int max_tiles(const WlMoeLayer& L, int64_t T, int cap, int gemv_max) {
     return static_cast<int>(routed + shared);
 }
 
+// The most tokens an expert averages for the small tiles. Q4_K / Q6_K layer, 256 experts, us with small / large tiles:
+// 1000 tokens (31 each) 294 / 399, 1500 315 / 410, 2000 (62) 406 / 459, 2800 (87) 486 / 485, 4096 (128) 618 / 520.
+constexpr int64_t kSmallTileAvg = 64;
+
 // 256-row slabs per down workgroup: several when there are enough tiles to fill the GPU with fewer workgroups, so
 // that each pays its pipeline start (and, with inter <= 512, its activation staging) once for several slabs.
 // Up to kDownFewTokens tokens (batched decode) always two: the grid is sized by the tile bound, most of its
@@ -1044,6 +1155,7 @@ static int down_slabs(const WlMoeLayer& L, int64_t T) {
     const int nslab = L.hidden / 256;
     const int64_t tiles = (T * L.top_k + kDownTileTokens - 1) / kDownTileTokens;  // about the full tiles
     if (T <= kDownFewTokens && nslab % 2 == 0) return 2;
+    if (tile_caps(L, T).down == kSmallTileTokens && nslab % 2 == 0) return 2;  // of 128 rows; 1, 4: 310, 301 us for 294
     int p = 1;
     while (p < kDownSlabsMax && nslab % (2 * p) == 0 && tiles * nslab / (2 * p) >= kDownMinGroups) p *= 2;
     return p;
@@ -1063,7 +1175,7 @@ static PrefillArgs prefill_args(const WlMoeLayer& L, int64_t T, const Workspace&
     a.tiles = w.tiles;
     a.n_tiles = w.n_tiles;
     a.tiles_down = w.tiles_down;
-    a.n_tiles_down = w.n_tiles + 1;
+    a.n_tiles_down = w.tiles_down == w.tiles ? w.n_tiles : w.n_tiles + 1;
     a.h16 = w.h16;
     a.h_sh16 = w.h_sh16;
     // the routed outputs share the fp32 buffer with the GEMV experts' outputs: position pos's bf16 row fills the
@@ -1080,6 +1192,11 @@ static PrefillArgs prefill_args(const WlMoeLayer& L, int64_t T, const Workspace&
     a.nslab_gate_up = (inter_max + 127) / 128;
     a.down_slabs = down_slabs(L, T);
     return a;
+}
+
+TileCaps tile_caps(const WlMoeLayer& L, int64_t T) {
+    if (T * L.top_k <= kSmallTileAvg * L.n_experts) return {kSmallTileTokens, kSmallTileTokens};
+    return {L.gate_up_type == WL_TYPE_Q4_K ? kTileTokens : kDownTileTokens, kDownTileTokens};
 }
 
 static int tiles8(const WlMoeLayer& L, int64_t T, int cap, int gemv_max) {
@@ -1110,7 +1227,7 @@ template <int KQ>
 static int launch_gate_up_ks(const WlMoeLayer& L, int64_t T, PrefillArgs a, int gemv_max, hipStream_t s) {
     const int inter_max = a.sh_inter > a.inter ? a.sh_inter : a.inter;
     a.nslab_gate_up = (inter_max + ks_slab<KQ>() - 1) / ks_slab<KQ>();
-    const dim3 grid(static_cast<unsigned>(a.nslab_gate_up * tiles8(L, T, kTileTokens, gemv_max)));
+    const dim3 grid(static_cast<unsigned>(a.nslab_gate_up * tiles8(L, T, tile_caps(L, T).gate_up, gemv_max)));
     if (L.gate_up_type == WL_TYPE_Q4_K)
         k_gemm_gate_up_ks<WL_TYPE_Q4_K, KQ><<<grid, kGemmThreads, 0, s>>>(a);
     else
@@ -1127,14 +1244,16 @@ int launch_mfma_gate_up(const WlMoeLayer& L, int64_t T, const Workspace& w, int 
     if (ks_eligible(L, T))
         return with_gemv ? launch_gate_up_ks<kKsGateUpBeside>(L, T, a, gemv_max, s)
                          : launch_gate_up_ks<kKsGateUp>(L, T, a, gemv_max, s);
-    if (L.gate_up_type == WL_TYPE_Q4_K)
-        k_gemm_gate_up<WL_TYPE_Q4_K, kTileTokens>
-            <<<dim3(static_cast<unsigned>(a.nslab_gate_up * tiles8(L, T, kTileTokens, gemv_max))), kGemmThreads, 0,
-               s>>>(a);
+    const int cap = tile_caps(L, T).gate_up;
+    if (cap == kSmallTileTokens) a.nslab_gate_up *= kGemmWaves / kSmallWaves;
+    const dim3 grid(static_cast<unsigned>(a.nslab_gate_up * tiles8(L, T, cap, gemv_max)));
+    const bool q4 = L.gate_up_type == WL_TYPE_Q4_K;
+    if (cap == kSmallTileTokens)
+        (q4 ? k_gemm_gate_up<WL_TYPE_Q4_K, kSmallTileTokens> : k_gemm_gate_up<WL_TYPE_Q6_K, kSmallTileTokens>)
+            <<<grid, 64 * kSmallWaves, 0, s>>>(a);
     else
-        k_gemm_gate_up<WL_TYPE_Q6_K, kDownTileTokens>
-            <<<dim3(static_cast<unsigned>(a.nslab_gate_up * tiles8(L, T, kDownTileTokens, gemv_max))), kGemmThreads,
-               0, s>>>(a);
+        (q4 ? k_gemm_gate_up<WL_TYPE_Q4_K, kTileTokens> : k_gemm_gate_up<WL_TYPE_Q6_K, kDownTileTokens>)
+            <<<grid, kGemmThreads, 0, s>>>(a);
     return launch_status();
 }
 
@@ -1144,18 +1263,23 @@ int launch_mfma_down(const WlMoeLayer& L, int64_t T, const Workspace& w, int gem
     PrefillArgs a = prefill_args(L, T, w);
     a.skip = skip;
     if (ks_eligible(L, T)) {
-        const dim3 grid(static_cast<unsigned>(L.hidden / kKsRows * tiles8(L, T, kDownTileTokens, gemv_max)));
+        const dim3 grid(static_cast<unsigned>(L.hidden / kKsRows * tiles8(L, T, tile_caps(L, T).down, gemv_max)));
         if (L.down_type == WL_TYPE_Q4_K)
             k_gemm_down_ks<WL_TYPE_Q4_K, kKsDown><<<grid, kGemmThreads, 0, s>>>(a);
         else
             k_gemm_down_ks<WL_TYPE_Q6_K, kKsDown><<<grid, kGemmThreads, 0, s>>>(a);
         return launch_status();
     }
-    const dim3 g2(static_cast<unsigned>(L.hidden / 256 / a.down_slabs * tiles8(L, T, kDownTileTokens, gemv_max)));
-    if (L.down_type == WL_TYPE_Q4_K)
-        k_gemm_down<WL_TYPE_Q4_K><<<g2, kGemmThreads, 0, s>>>(a);
+    const int cap = tile_caps(L, T).down;
+    const int rows = cap == kSmallTileTokens ? gemm_rows<kSmallTileTokens>() : gemm_rows<kDownTileTokens>();
+    const dim3 g2(static_cast<unsigned>(L.hidden / rows / a.down_slabs * tiles8(L, T, cap, gemv_max)));
+    const bool q4 = L.down_type == WL_TYPE_Q4_K;
+    if (cap == kSmallTileTokens)
+        (q4 ? k_gemm_down<WL_TYPE_Q4_K, kSmallTileTokens> : k_gemm_down<WL_TYPE_Q6_K, kSmallTileTokens>)
+            <<<g2, 64 * kSmallWaves, 0, s>>>(a);
     else
-        k_gemm_down<WL_TYPE_Q6_K><<<g2, kGemmThreads, 0, s>>>(a);
+        (q4 ? k_gemm_down<WL_TYPE_Q4_K, kDownTileTokens> : k_gemm_down<WL_TYPE_Q6_K, kDownTileTokens>)
+            <<<g2, kGemmThreads, 0, s>>>(a);
     return launch_status();
 }
 
@@ -1177,9 +1301,9 @@ int launch_linear(int type, const uint8_t* w, int rows, int k, const uint16_t* x
     const int tiles = static_cast<int>((T + kDownTileTokens - 1) / kDownTileTokens);
     const dim3 grid(static_cast<unsigned>(rows / 256 * ((tiles + kXcds - 1) / kXcds * kXcds)));
     if (type == WL_TYPE_Q4_K)
-        k_gemm_down<WL_TYPE_Q4_K><<<grid, kGemmThreads, 0, s>>>(a);
+        k_gemm_down<WL_TYPE_Q4_K, kDownTileTokens><<<grid, kGemmThreads, 0, s>>>(a);
     else
-        k_gemm_down<WL_TYPE_Q6_K><<<grid, kGemmThreads, 0, s>>>(a);
+        k_gemm_down<WL_TYPE_Q6_K, kDownTileTokens><<<grid, kGemmThreads, 0, s>>>(a);
     return launch_status();
 }
 
