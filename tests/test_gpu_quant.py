@@ -172,6 +172,25 @@ def test_linear_mfma(hip, name, rows, k, tokens):
     assert err < 4e-3, err
 
 
+@pytest.mark.parametrize("name,rows,k,tokens", [
+    ("Q4_K", 256, 768, 9), ("Q6_K", 768, 1280, 65), ("Q4_K", 2304, 2048, 200), ("Q6_K", 256, 1024, 449),  # K 4 ways
+    ("Q6_K", 512, 512, 17), ("Q4_K", 768, 512, 500), ("Q6_K", 2048, 1280, 700),                           # K 2 ways
+    ("Q4_K", 4096, 256, 130), ("Q6_K", 4096, 1280, 1000), ("Q4_K", 4096, 768, 640),                   # 64-token tiles
+    ("Q6_K", 4096, 512, 1300)])                                                                      # 128-token tiles
+def test_linear_mfma_forms(hip, name, rows, k, tokens):
+    """Each kernel of wl_linear at its edges: block counts that do not divide into the K split, fewer than 8 token
+    tiles and 8 or more, row slabs that do not fill the 8 XCDs, a last tile of 1, 8, 17 and 64 tokens. Bound: bf16's
+    half ulp on the output (2^-9 of its value) plus the fp32 sums' rounding (k 2^-24 of sum |w x|)."""
+    rng = np.random.default_rng(rows + k + tokens)
+    w = synth.matrix(rng, name, rows, k)
+    x = rng.standard_normal((tokens, k)).astype(np.float32)
+    y = hip.linear_mfma(dev(w).reshape(-1), name, (rows, k), torch.from_numpy(x).cuda()).float().cpu().numpy()
+    wb = q.round_bf16(q.dequantize_matrix(w, name, rows, k)).astype(np.float64)
+    xb = q.round_bf16(x).astype(np.float64)
+    ref, size = xb @ wb.T, np.abs(xb) @ np.abs(wb).T
+    assert (np.abs(y - ref) <= 2.0 ** -8 * np.abs(ref) + k * 2.0 ** -24 * size).all()
+
+
 def test_linear_mfma_rejects(hip):
     w = torch.zeros(255 * 144, dtype=torch.uint8, device="cuda")
     x = torch.zeros(16, 256, device="cuda")

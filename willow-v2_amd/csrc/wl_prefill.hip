@@ -818,6 +818,30 @@ __device__ __forceinline__ void slab_tile(int nslab, int& slab, int& tile) {
     tile = (i / nslab) * kXcds + x;
 }
 
+// wl_linear's token tile and row slab of a workgroup; false when it has none. From 8 tiles on as slab_tile; fewer would
+// leave most of a grid padded to 8 tiles empty, so there the slabs are dealt to the XCDs, each slab's tiles one after
+// another on one of them (linear_grid sizes the grid either way).
+__host__ __device__ inline int round_up8(int v) { return (v + kXcds - 1) / kXcds * kXcds; }
+template <int TILE>
+__device__ __forceinline__ bool linear_tile(int tokens, int nslab, int& slab, int4& tile) {
+    const int tiles = (tokens + TILE - 1) / TILE;
+    int ti;
+    if (tiles >= kXcds) {
+        slab_tile(nslab, slab, ti);
+    } else {
+        const int b = static_cast<int>(blockIdx.x), i = b / kXcds;
+        slab = i / tiles * kXcds + b % kXcds;
+        ti = i % tiles;
+    }
+    const int p = ti * TILE;
+    tile = make_int4(0, p, min(TILE, tokens - p), 0);
+    return slab < nslab && p < tokens;
+}
+static unsigned linear_grid(int nslab, int64_t tokens, int cap) {
+    const int tiles = static_cast<int>((tokens + cap - 1) / cap);
+    return static_cast<unsigned>(tiles >= kXcds ? nslab * round_up8(tiles) : round_up8(nslab) * tiles);
+}
+
 // gate_up: slab = 128-row slab of the intermediate dim; wavefront w: gate rows j0 + 16r + lr (r < kRT / 2)
 // and the matching up rows inter + j0 + ... (r >= kRT / 2), j0 = 128 slab + 8 kRT w. Epilogue h = silu(g) * u -> bf16.
 // TILE is tile_caps().gate_up: kTileTokens, kDownTileTokens for Q6_K rows (whose larger row state leaves no registers
@@ -879,13 +903,11 @@ __global__ __launch_bounds__(64 * gemm_wg_waves<TILE>(), TILE == kSmallTileToken
     if (a.skip && *a.skip) return;
     int group, ti;
     constexpr int kRows = gemm_rows<TILE>();
-    slab_tile(a.H / kRows / a.down_slabs, group, ti);
     int4 tile;
-    if (a.dense_tokens > 0) {  // wl_linear: token tile ti of one matrix
-        const int p = ti * TILE;
-        if (p >= a.dense_tokens) return;
-        tile = make_int4(0, p, min(TILE, a.dense_tokens - p), 0);
+    if (a.dense_tokens > 0) {  // wl_linear: one matrix
+        if (!linear_tile<TILE>(a.dense_tokens, a.H / kRows, group, tile)) return;
     } else {
+        slab_tile(a.H / kRows / a.down_slabs, group, ti);
         if (ti >= a.n_tiles_down[0]) return;
         tile = a.tiles_down[ti];
     }
@@ -946,14 +968,14 @@ __device__ __forceinline__ void gemm_ksplit(uint8_t* lds, floatx4 (&acc)[kRT][kK
     const uint32_t col = 16u * static_cast<uint32_t>((lane & 31) ^ ((2 * wv + half) & swizzle<TYPE>()));
     const uint32_t lds0 = lds_address(lds);
     const BAddr ba = b_addr<TYPE>(lr, q);
-    const int nphase = nblocks / KQ;
+    const int nphase = (nblocks + KQ - 1) / KQ;  // the last phase may hold fewer chunks
     RowState<TYPE> rs[kRT], nx[kRT];
 #pragma unroll
-    for (int r = 0; r < kRT; r++) rs[r].fetch(row_ptr(r, lr) + static_cast<int64_t>(kq) * BlockInfo<TYPE>::bytes, q);
+    for (int r = 0; r < kRT; r++) rs[r].fetch(row_ptr(r, lr) + static_cast<int64_t>(min(kq, nblocks - 1)) * BlockInfo<TYPE>::bytes, q);
     bf16x8 a0[kRT], a1[kRT], b[NT];
     for (int p = 0; p < nphase; p++) {
         if (p > 0) __syncthreads();  // every wavefront is done with the previous phase's chunks
-        for (int c = 0; c < KQ; c++)
+        for (int c = 0; c < min(KQ, nblocks - p * KQ); c++)
             stage_async<kKsTile, NT>(lds0 + c * kChunk, src + static_cast<int64_t>(p * KQ + c) * kTileRowBytes, rowtab,
                                      col, wv, half);
         wait_stage();  // the phase's chunks and this wavefront's row states have landed
@@ -961,8 +983,10 @@ __device__ __forceinline__ void gemm_ksplit(uint8_t* lds, floatx4 (&acc)[kRT][kK
         if (p + 1 < nphase) {
 #pragma unroll
             for (int r = 0; r < kRT; r++)
-                nx[r].fetch(row_ptr(r, lr) + static_cast<int64_t>((p + 1) * KQ + kq) * BlockInfo<TYPE>::bytes, q);
+                nx[r].fetch(row_ptr(r, lr) + static_cast<int64_t>(min((p + 1) * KQ + kq, nblocks - 1)) *
+                                                 BlockInfo<TYPE>::bytes, q);
         }
+        if (p * KQ + kq >= nblocks) break;  // the last phase, no chunk left for this wavefront
         const uint8_t* buf = lds + kq * kChunk;
         read_b<TYPE, NT, 0>(buf, ba, b);
 #pragma unroll
@@ -1079,9 +1103,14 @@ __global__ __launch_bounds__(kGemmThreads) void k_gemm_down_ks(PrefillArgs a) {
     constexpr int kRows = 16 * kRT * kGemmWaves / KQ;
     if (a.skip && *a.skip) return;
     int group, ti;
-    slab_tile(a.H / kRows, group, ti);
-    if (ti >= a.n_tiles_down[0]) return;
-    const int4 tile = a.tiles_down[ti];
+    int4 tile;
+    if (a.dense_tokens > 0) {  // wl_linear: one matrix
+        if (!linear_tile<kKsTile>(a.dense_tokens, a.H / kRows, group, tile)) return;
+    } else {
+        slab_tile(a.H / kRows, group, ti);
+        if (ti >= a.n_tiles_down[0]) return;
+        tile = a.tiles_down[ti];
+    }
     const bool sh = tile.x == a.E;
     const int inter = sh ? a.sh_inter : a.inter;
     const int wv = static_cast<int>(threadIdx.x >> 6), rg = wv / KQ, kq = wv % KQ;
@@ -1208,7 +1237,9 @@ static int tiles8(const WlMoeLayer& L, int64_t T, int cap, int gemv_max) {
 constexpr int kKsGateUp = 4, kKsGateUpBeside = 2, kKsDown = 2;
 template <int KQ>
 constexpr int ks_slab() { return 16 * kGemmWaves / KQ; }  // gate rows per k_gemm_gate_up_ks<., KQ> workgroup
-constexpr int kKsRows = 16 * kRT * kGemmWaves / kKsDown;  // output rows per k_gemm_down_ks workgroup
+template <int KQ>
+constexpr int ks_rows() { return 16 * kRT * kGemmWaves / KQ; }  // output rows per k_gemm_down_ks workgroup
+constexpr int kKsRows = ks_rows<kKsDown>();
 
 // Whether a call runs the K-split kernels: at most kKsTile tokens (so every tile holds at most that many), and
 // shapes whose block counts divide into the ways and whose rows divide into the workgroups' row sets (the larger
@@ -1283,6 +1314,15 @@ int launch_mfma_down(const WlMoeLayer& L, int64_t T, const Workspace& w, int gem
     return launch_status();
 }
 
+// The kernel of a wl_linear call, by how many workgroups it would run. While one round of the CUs takes them (a K-split
+// workgroup fills one), the K loop split 4 ways, or 2 with up to two blocks a row, is the shortest chain; then 64-token
+// tiles, three workgroups a CU; then the 128-token tiles, which decode each weight half as often. us by kernel, and
+// before (128-token tiles always): Q4_K 4096 x 2048, 200 tokens, 4 ways 12.5, 64-token tiles 24.5, before 38.5; 500
+// tokens 4 ways 25.3 (two rounds), 2 ways 20.8, 64-token 25.1, before 39.2; 1000 tokens 2 ways 37.6, 64-token 28.6,
+// before 40.8; 2048 tokens (1024 workgroups) 64-token 57.1, 128-token 44.3. Q6_K 4096 x 512, 1500 tokens (768) 20.8
+// and 20.7.
+constexpr int64_t kLinearKsGroups = 256, kLinearSmallGroups = 640;
+
 // y[t, :] = W x[t, :] for a single quantized matrix on the down GEMM: bf16 operands (x as given, W's exact values
 // rounded to bf16 in registers), fp32 accumulation, bf16 output. rows and k are multiples of 256.
 int launch_linear(int type, const uint8_t* w, int rows, int k, const uint16_t* x, int64_t T, uint16_t* y,
@@ -1298,12 +1338,23 @@ int launch_linear(int type, const uint8_t* w, int rows, int k, const uint16_t* x
     a.E = 1;  // the one matrix is expert 0, never the shared slot
     a.down_slabs = 1;
     a.dense_tokens = static_cast<int>(T);
-    const int tiles = static_cast<int>((T + kDownTileTokens - 1) / kDownTileTokens);
-    const dim3 grid(static_cast<unsigned>(rows / 256 * ((tiles + kXcds - 1) / kXcds * kXcds)));
-    if (type == WL_TYPE_Q4_K)
-        k_gemm_down<WL_TYPE_Q4_K, kDownTileTokens><<<grid, kGemmThreads, 0, s>>>(a);
+    const bool q4 = type == WL_TYPE_Q4_K;
+    const int64_t tiles = (T + kSmallTileTokens - 1) / kSmallTileTokens;
+    static_assert(kKsTile == kSmallTileTokens, "");
+    auto groups = [&](int wg_rows) { return tiles * (rows / wg_rows); };
+    auto grid = [&](int wg_rows, int cap) { return dim3(linear_grid(rows / wg_rows, T, cap)); };
+    if (k > 2 * kQK && groups(ks_rows<4>()) <= kLinearKsGroups)
+        (q4 ? k_gemm_down_ks<WL_TYPE_Q4_K, 4> : k_gemm_down_ks<WL_TYPE_Q6_K, 4>)
+            <<<grid(ks_rows<4>(), kKsTile), kGemmThreads, 0, s>>>(a);
+    else if (k > kQK && groups(ks_rows<2>()) <= kLinearKsGroups)
+        (q4 ? k_gemm_down_ks<WL_TYPE_Q4_K, 2> : k_gemm_down_ks<WL_TYPE_Q6_K, 2>)
+            <<<grid(ks_rows<2>(), kKsTile), kGemmThreads, 0, s>>>(a);
+    else if (groups(gemm_rows<kSmallTileTokens>()) <= kLinearSmallGroups)
+        (q4 ? k_gemm_down<WL_TYPE_Q4_K, kSmallTileTokens> : k_gemm_down<WL_TYPE_Q6_K, kSmallTileTokens>)
+            <<<grid(gemm_rows<kSmallTileTokens>(), kSmallTileTokens), 64 * kSmallWaves, 0, s>>>(a);
     else
-        k_gemm_down<WL_TYPE_Q6_K, kDownTileTokens><<<grid, kGemmThreads, 0, s>>>(a);
+        (q4 ? k_gemm_down<WL_TYPE_Q4_K, kDownTileTokens> : k_gemm_down<WL_TYPE_Q6_K, kDownTileTokens>)
+            <<<grid(gemm_rows<kDownTileTokens>(), kDownTileTokens), kGemmThreads, 0, s>>>(a);
     return launch_status();
 }
 
