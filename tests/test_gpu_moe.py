@@ -480,3 +480,19 @@ def test_pre_norm_residual(hip, c2, layer_c2, c2_norm_weight, T, weighted, resid
     want = (x + y_plain) if residual else y_plain
     np.testing.assert_array_equal(y.view(np.uint32), want.view(np.uint32))
     check_layer(hip, c2, layer_c2, xn, f"pre_norm T={T}")
+
+
+@pytest.mark.parametrize("hidden,T,weighted", [(256, 2, True), (1024, 8, True), (1024, 15, False), (2048, 16, True),
+                                                 (2048, 17, True), (4096, 40, True)])
+def test_pre_norm_in_router(hip, hidden, T, weighted):
+    """The router's own normalization (2 to 64 tokens): one round of 32 segments, part of one and two, token tiles full,
+    short and just begun; bit for bit the plain layer on the oracle's rms_norm(x), which shares no code with it."""
+    lw = synth.moe_layer(90, hidden=hidden, inter=256, shared_inter=256, experts=40, top_k=4)
+    w = (np.random.default_rng(91).standard_normal(hidden) * 0.1).astype(np.float32) if weighted else None
+    layer = hip.MoELayer.from_host(lw, pre_norm=True, norm_weight=w, norm_eps=1e-6, residual=True)
+    x = synth.tokens(92, T, hidden) * np.float32(3.0)
+    y, ids, wts = run_layer(hip, layer, x)
+    y_plain, ids_plain, wts_plain = run_layer(hip, hip.MoELayer.from_host(lw), moe_ref.rms_norm(x, w, 1e-6))
+    np.testing.assert_array_equal(ids, ids_plain)
+    np.testing.assert_array_equal(wts.view(np.uint32), wts_plain.view(np.uint32))
+    np.testing.assert_array_equal(y.view(np.uint32), (x + y_plain).view(np.uint32))

@@ -196,12 +196,68 @@ __global__ __launch_bounds__(256) void k_topk(const float* __restrict__ logits, 
 // and no partial sum inside the workgroup. k_topk_parts then adds each row's partials in segment order and the
 // bias: the order of router_row, so the logits are the same bits. With xb, the first row tile's workgroups also
 // store the tokens' values as bf16.
+//
+//
+// NORM (WL_MOE_PRE_NORM): x is normalized as it is staged. A workgroup's 8 wavefronts first take the sums of squares
+// of its 16 tokens (k_rms_norm's order, so the same bits), each token's row read once, contiguously, and cut into
+// segments through the wavefront's staging area; the first row tile's workgroups store the normalized values for the
+// expert kernels. As a launch of its own the norm took 7.7 us of a 5-token layer (its lanes read 256 bytes apart, 64
+// lines a load; the same reads in here saved nothing): layer 67.9 -> 63.6 us at 5 tokens, 47 -> 42.8 at 2.
+struct NormIn {
+    const float* w;  // nullable
+    float eps;
+    float* xn;
+};
+
+// The sum of squares of x[0, H) in router_row's order (router_row(x, x)), by one wavefront; `area`: 32 kSqPitch floats
+// of LDS of its own. Every lane returns it.
+constexpr int kSqPitch = kRouterSeg + 4;
+static_assert(32 * kSqPitch <= 2 * kRsTile, "row_square_sum uses a wavefront's staging area");
+__device__ __forceinline__ float row_square_sum(const float* __restrict__ x, int H, int lane, float* area) {
+    const int nseg = H / kRouterSeg;
+    float total = 0.0f;
+    for (int j = 0; 32 * j < nseg; j++) {
+        float4 v[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) {  // float4 lane + 64 i of these 32 segments
+            const int at = 32 * kRouterSeg * j + 4 * (lane + 64 * i);
+            v[i] = at < H ? *reinterpret_cast<const float4*>(x + at) : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int f = lane + 64 * i;
+            *reinterpret_cast<float4*>(area + (f >> 4) * kSqPitch + 4 * (f & 15)) = v[i];
+        }
+        lane_sync();
+        float4 q[kRouterSeg / 4];
+#pragma unroll
+        for (int i = 0; i < kRouterSeg / 4; i++)
+            q[i] = *reinterpret_cast<const float4*>(area + (lane & 31) * kSqPitch + 4 * i);
+        __builtin_amdgcn_sched_barrier(0);
+        float p = 0.0f;
+#pragma unroll
+        for (int i = 0; i < kRouterSeg / 4; i++) {
+            p = __builtin_fmaf(q[i].x, q[i].x, p);
+            p = __builtin_fmaf(q[i].y, q[i].y, p);
+            p = __builtin_fmaf(q[i].z, q[i].z, p);
+            p = __builtin_fmaf(q[i].w, q[i].w, p);
+        }
+        for (int sl = 0; sl < 32 && 32 * j + sl < nseg; sl++) {  // in segment order
+            const float ps = __builtin_bit_cast(
+                float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, p), sl));
+            total = j == 0 && sl == 0 ? ps : __fadd_rn(total, ps);
+        }
+        lane_sync();  // the area is rewritten
+    }
+    return total;
+}
+template <bool NORM>
 __global__ __launch_bounds__(64 * kRsWaves) void k_router_parts(const float* __restrict__ x,
                                                                 const float* __restrict__ w,
                                                                 const float* __restrict__ shared_gate, int T,
                                                                 int H, int E, float* __restrict__ parts,
                                                                 uint16_t* __restrict__ xb,
-                                                                uint32_t* __restrict__ topk_done) {
+                                                                uint32_t* __restrict__ topk_done, NormIn norm) {
     __shared__ __attribute__((aligned(16))) float stage[kRsWaves][2][kRsTile];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     // the count k_topk_group (next on this stream) starts from: zeroed here by every call, so a workspace whose
@@ -211,17 +267,39 @@ __global__ __launch_bounds__(64 * kRsWaves) void k_router_parts(const float* __r
     const int t0 = blockIdx.x * 16, r0 = blockIdx.y * 16;
     const int rows = E + (shared_gate ? 1 : 0);
     const int seg = static_cast<int>(blockIdx.z) * kRsWaves + wv;
-    if (seg >= H / kRouterSeg) return;  // the wavefront alone: nothing below synchronizes the workgroup
+    const bool have_seg = seg < H / kRouterSeg;
+    __shared__ float inv[16];
+    if constexpr (!NORM) {
+        if (!have_seg) return;  // the wavefront alone: nothing below synchronizes the workgroup
+    }
     // float4 f = lane + 64 i (i < 4) holds values 4 (f % 16) .. + 3 of the segment for token / row f / 16
     float4 xn[4], wn[4];
+    if (!NORM || have_seg) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int f = lane + 64 * i, rr = f >> 4, c4 = 4 * (f & 15);
-        const int t = t0 + rr, r = r0 + rr;
-        xn[i] = *reinterpret_cast<const float4*>(x + static_cast<int64_t>(t < T ? t : T - 1) * H + seg * kRouterSeg +
-                                                 c4);
-        const float* wr = r < rows ? (r < E ? w + static_cast<int64_t>(r) * H : shared_gate) : nullptr;
-        wn[i] = wr ? *reinterpret_cast<const float4*>(wr + seg * kRouterSeg + c4) : make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int i = 0; i < 4; i++) {
+            const int f = lane + 64 * i, rr = f >> 4, c4 = 4 * (f & 15);
+            const int t = t0 + rr, r = r0 + rr;
+            xn[i] = *reinterpret_cast<const float4*>(x + static_cast<int64_t>(t < T ? t : T - 1) * H + seg * kRouterSeg +
+                                                     c4);
+            const float* wr = r < rows ? (r < E ? w + static_cast<int64_t>(r) * H : shared_gate) : nullptr;
+            wn[i] = wr ? *reinterpret_cast<const float4*>(wr + seg * kRouterSeg + c4) : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    }
+    if constexpr (NORM) {
+        for (int u = wv; u < 16 && t0 + u < T; u += kRsWaves) {
+            const float sq = row_square_sum(x + static_cast<int64_t>(t0 + u) * H, H, lane, stage[wv][0]);
+            if (lane == 0) inv[u] = norm_inv(sq, H, norm.eps);
+        }
+        __syncthreads();
+        if (!have_seg) return;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int f = lane + 64 * i, rr = f >> 4, at = seg * kRouterSeg + 4 * (f & 15);
+            const float4 g = norm.w ? *reinterpret_cast<const float4*>(norm.w + at) : make_float4(0.f, 0.f, 0.f, 0.f);
+            xn[i] = norm_apply(xn[i], norm.w != nullptr, g, inv[min(rr, T - 1 - t0)]);
+            if (blockIdx.y == 0 && t0 + rr < T)
+                *reinterpret_cast<float4*>(norm.xn + static_cast<int64_t>(t0 + rr) * H + at) = xn[i];
+        }
     }
     float* sa = stage[wv][0];
     float* sb = stage[wv][1];
@@ -1431,15 +1509,17 @@ static int launch_topk(const WlMoeLayer& L, const float* logits, int64_t T, int3
 }
 
 // Router and top-k of a call of 2 .. kRouterPartsMaxT tokens: k_router_parts, then k_topk_parts.
+// With norm, x is the layer's input and the normalized rows go to w.xn.
 static int launch_router_parts(const WlMoeLayer& L, const float* x, int64_t T, const Workspace& w, uint16_t* xb,
-                               hipStream_t s) {
+                               bool norm, hipStream_t s) {
     const float* shared_gate = (L.shared_gate_up && L.shared_gate) ? L.shared_gate : nullptr;
     const int rows = L.n_experts + (shared_gate ? 1 : 0);
     const int nseg = L.hidden / kRouterSeg;
-    k_router_parts<<<dim3(static_cast<unsigned>((T + 15) / 16), static_cast<unsigned>((rows + 15) / 16),
-                          static_cast<unsigned>((nseg + kRsWaves - 1) / kRsWaves)),
-                     64 * kRsWaves, 0, s>>>(x, L.router, shared_gate, static_cast<int>(T), L.hidden, L.n_experts,
-                                            w.parts, xb, w.sync + kTopkDone);
+    auto kernel = norm ? k_router_parts<true> : k_router_parts<false>;
+    const dim3 grid(static_cast<unsigned>((T + 15) / 16), static_cast<unsigned>((rows + 15) / 16),
+                    static_cast<unsigned>((nseg + kRsWaves - 1) / kRsWaves));
+    kernel<<<grid, 64 * kRsWaves, 0, s>>>(x, L.router, shared_gate, static_cast<int>(T), L.hidden, L.n_experts, w.parts,
+                                          xb, w.sync + kTopkDone, NormIn{L.norm_weight, L.norm_eps, w.xn});
     return launch_status();
 }
 
@@ -1767,7 +1847,12 @@ static int run_layer(const WlMoeLayer* layer, const float* x, int64_t tokens, fl
     auto mark = record;
     mark(0);
     const float* resid = (L.flags & WL_MOE_RESIDUAL) ? x : nullptr;
-    if (L.flags & WL_MOE_PRE_NORM) {  // every stage below runs on the normalized input
+    // every stage below runs on the normalized input; up to kRouterPartsMaxT tokens the router makes it
+    const float* router_x = x;
+    const bool norm_in_router = (L.flags & WL_MOE_PRE_NORM) && router_parts(tokens);
+    if (norm_in_router) {
+        x = w.xn;
+    } else if (L.flags & WL_MOE_PRE_NORM) {
         k_rms_norm<<<static_cast<unsigned>((tokens + 3) / 4), 256, 0, s>>>(x, L.norm_weight, L.norm_eps,
                                                                            static_cast<int>(tokens), L.hidden, w.xn);
         x = w.xn;
@@ -1796,7 +1881,7 @@ static int run_layer(const WlMoeLayer* layer, const float* x, int64_t tokens, fl
     }
     const bool starve = (L.flags & WL_MOE_TEST_STARVE) != 0;
     if (router_parts(tokens)) {
-        rc = launch_router_parts(L, x, tokens, w, mfma ? w.xb : nullptr, s);
+        rc = launch_router_parts(L, router_x, tokens, w, mfma ? w.xb : nullptr, norm_in_router, s);
         if (rc) return rc;
         mark(1);
         // the grouping in the same launch (mark 3 follows mark 2 at once)
