@@ -44,6 +44,33 @@ def test_dequant_bit_exact(hip, name, rows, k, dtype):
                                   expect.view(np.uint16 if dtype == "bf16" else np.uint32))
 
 
+@pytest.mark.parametrize("name", ["Q4_K", "Q6_K"])
+@pytest.mark.parametrize("pad", [0, 96])
+def test_dequant_nonfinite_and_strided(hip, name, pad):
+    """bf16 values are the fp32 ones rounded to nearest even, NaN as 0x7FC0, also where a block's scale is infinite or
+    NaN (the lanes that leave the packed conversion), with dense rows and with padding between them."""
+    rows, k = 5, 768
+    w = synth.matrix(np.random.default_rng(77), name, rows, k).reshape(rows, -1)
+    per, at = (144, 0) if name == "Q4_K" else (210, 208)
+    for r, bits in ((1, 0x7C00), (2, 0xFC00), (3, 0x7E01)):  # inf, -inf, NaN with a payload, in block r - 1 of row r
+        w[r, per * (r - 1) + at:per * (r - 1) + at + 2] = np.frombuffer(np.uint16(bits).tobytes(), np.uint8)
+    stride = w.shape[1] + pad
+    padded = np.zeros((rows, stride), np.uint8)
+    padded[:, :w.shape[1]] = w
+    raw = dev(padded)
+    out = {}
+    for code, dtype in ((hip.DTYPE_F32, torch.float32), (hip.DTYPE_BF16, torch.bfloat16)):
+        out[code] = torch.empty(rows, k, dtype=dtype, device="cuda")
+        assert hip.library().wl_dequant(hip.TYPE_IDS[name], raw.data_ptr(), rows, k, stride, code, out[code].data_ptr(),
+                                        torch.cuda.current_stream().cuda_stream) == 0
+    f = out[hip.DTYPE_F32].cpu().numpy()
+    ok = np.isfinite(f)
+    assert not ok.all() and ok[0].all() and ok[4].all()
+    u = f.view(np.uint32).astype(np.uint64)
+    want = np.where(np.isnan(f), 0x7FC0, (u + 0x7FFF + ((u >> 16) & 1)) >> 16).astype(np.uint16)
+    np.testing.assert_array_equal(out[hip.DTYPE_BF16].cpu().view(torch.int16).numpy().view(np.uint16), want)
+
+
 def test_gemv_config0(hip):
     """The 512x2048 Q4_K GEMV (seed 0)."""
     case = synth.gemv_case(0)
