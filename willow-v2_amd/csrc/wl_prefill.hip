@@ -9,9 +9,10 @@
 //   k_router_mfma    logits for many tokens in the router's fixed order (64-value FMA segments, added left to
 //                    right); also writes x as bf16 (the small-batch router in wl_moe.hip does the same)
 //   (sort)           the sort's single-workgroup stage writes the tile lists (tile_list): per-expert tiles of
-//                    sorted positions, then the shared expert's, of at most 144 (gate_up) and 128 (down) tokens
-//   k_gemm_gate_up   per (tile, 128 intermediate rows): gate and up rows together, epilogue h = silu(g) * u -> bf16
-//   k_gemm_down      per (tile, 256 output rows): o = down h, fp32, by sorted position (combined by k_combine)
+//                    sorted positions, then the shared expert's, of at most 144 (gate_up) and 128 (down) tokens,
+//                    or of 64 for both when the experts average no more (tile_caps)
+//   k_gemm_gate_up   per (tile, 128 intermediate rows; 64 with small tiles): gate and up rows together, epilogue h = silu(g) * u -> bf16
+//   k_gemm_down      per (tile, 256 output rows; 128 with small tiles): o = down h, fp32, by sorted position (combined by k_combine)
 //
 // MFMA 16x16x32 bf16 operand layout (wave64): lane l holds A[l % 16][8 (l / 16) + i], B[8 (l / 16) + i][l % 16],
 // and C[4 (l / 16) + i][l % 16], i < 8 (A, B) or < 4 (C). A wavefront covers kRT row tiles x up to 9 token tiles.
