@@ -120,6 +120,21 @@ def test_gemv_forms(hip, name, rows, k, tokens):
     assert torch.equal(F.linear(odd, hip.GGMLWeight(raw, name, (rows, k))), y)  # x off a 16-byte boundary
 
 
+@pytest.mark.parametrize("name,rows,k", [("Q4_K", 512, 2048), ("Q6_K", 512, 2048), ("Q4_K", 40, 4096),
+                                         ("Q6_K", 24, 8704)])
+@pytest.mark.parametrize("tokens", [1, 8])
+def test_gemv_small_x(hip, name, rows, k, tokens):
+    """x 2^-110 gives y 2^-110 bit for bit: scaling by a power of two rounds the same while nothing is subnormal. x holds
+    all 24 bits and |x| is in [2^-6, 4), so every product and sum of a run is a multiple of 2^-139, a normal number or an
+    exact subnormal; a kernel that scales the products down further loses their low bits."""
+    rng = np.random.default_rng(rows + k + tokens)
+    raw = dev(synth.matrix(rng, name, rows, k)).reshape(-1)
+    x = rng.uniform(2.0 ** -6, 4.0, (tokens, k)) * rng.choice((-1.0, 1.0), (tokens, k))
+    x = torch.from_numpy(x.astype(np.float32)).cuda()
+    y = hip.gemv(raw, name, (rows, k), x)
+    assert torch.equal(hip.gemv(raw, name, (rows, k), x * 2.0 ** -110), y * 2.0 ** -110)
+
+
 def test_gemv_batch_and_combine(hip):
     """gate_up of 4 experts in one launch (gemv_batch), then down + weighted sum (gemv_combine), as
     Engine.batched_decode_experts drives them (engines/base.py:492-532)."""

@@ -7,50 +7,43 @@
 
 namespace wl {
 
-// A lane's two 16-value runs of a block as f16 pairs (values 0 and 2 of each packed word in e, 1 and 3 in o) whose
-// exponent bits are zero: v_fma_mix_f32 reads such a half as the subnormal q 2^-s, so no value is ever converted. The
-// pairs are made once per block and used for every token; a (the run's scale) carries the 2^s back, exactly.
+// A lane's two 16-value runs of a block as exact f16 pairs (values 0 and 2 of each packed word in e, 1 and 3 in o),
+// which v_fma_mix_f32 reads directly. A pair is one byte permute (each byte under 0x64: 1024 + q) and one packed
+// subtraction, made once per block and used for every token, in half the registers that fp32 values take. The values
+// are q itself, not q 2^-24 (the raw field as an f16 subnormal, one instruction less): products with |x| < 2^-102
+// would be fp32 subnormals and lose bits (|x| near 1e-36: error 6e-4).
 template <int TYPE>
 struct HalfRuns {
-    uint32_t e_lo[4], o_lo[4], e_hi[4], o_hi[4];
+    wl_f16x2 e_lo[4], o_lo[4], e_hi[4], o_hi[4];
     float a_lo, a_hi, b_lo, b_hi;
+    template <int FIRST>
+    static __device__ __forceinline__ wl_f16x2 pair(uint32_t w) {  // bytes FIRST and FIRST + 2
+        const uint32_t v = __builtin_amdgcn_perm(0x64646464u, w, FIRST == 0 ? 0x04020400u : 0x04030401u);
+        return __builtin_bit_cast(wl_f16x2, v) - static_cast<_Float16>(1024.0f);
+    }
     __device__ __forceinline__ void set(const RawLane<TYPE>& raw, int c) {
         Lane32 l;
-        if constexpr (TYPE == WL_TYPE_Q4_K) {
-            raw.unpack_mix(c, l);
+        raw.unpack(c, l);
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                e_lo[i] = l.lo[i] & 0x000F000Fu;
-                o_lo[i] = (l.lo[i] >> 8) & 0x000F000Fu;
-                e_hi[i] = l.lo[i] & 0x00F000F0u;
-                o_hi[i] = (l.lo[i] >> 8) & 0x00F000F0u;
-            }
-            a_lo = l.a_lo;
-            a_hi = l.a_hi;
-        } else {
-            raw.unpack(c, l);
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                e_lo[i] = l.lo[i] & 0x00FF00FFu;
-                o_lo[i] = (l.lo[i] >> 8) & 0x00FF00FFu;
-                e_hi[i] = l.hi[i] & 0x00FF00FFu;
-                o_hi[i] = (l.hi[i] >> 8) & 0x00FF00FFu;
-            }
-            a_lo = l.a_lo * 16777216.0f;
-            a_hi = l.a_hi * 16777216.0f;
+        for (int i = 0; i < 4; i++) {
+            e_lo[i] = pair<0>(l.lo[i]);
+            o_lo[i] = pair<1>(l.lo[i]);
+            e_hi[i] = pair<0>(l.hi[i]);
+            o_hi[i] = pair<1>(l.hi[i]);
         }
+        a_lo = l.a_lo;
+        a_hi = l.a_hi;
         b_lo = l.b_lo;
         b_hi = l.b_hi;
     }
-    static __device__ __forceinline__ float dot(const uint32_t (&e)[4], const uint32_t (&o)[4], const float4 (&x)[4]) {
+    static __device__ __forceinline__ float dot(const wl_f16x2 (&e)[4], const wl_f16x2 (&o)[4], const float4 (&x)[4]) {
         float s0 = 0.0f, s1 = 0.0f;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const wl_f16x2 he = __builtin_bit_cast(wl_f16x2, e[i]), ho = __builtin_bit_cast(wl_f16x2, o[i]);
-            s0 = __builtin_fmaf(static_cast<float>(he.x), x[i].x, s0);
-            s1 = __builtin_fmaf(static_cast<float>(ho.x), x[i].y, s1);
-            s0 = __builtin_fmaf(static_cast<float>(he.y), x[i].z, s0);
-            s1 = __builtin_fmaf(static_cast<float>(ho.y), x[i].w, s1);
+            s0 = __builtin_fmaf(static_cast<float>(e[i].x), x[i].x, s0);
+            s1 = __builtin_fmaf(static_cast<float>(o[i].x), x[i].y, s1);
+            s0 = __builtin_fmaf(static_cast<float>(e[i].y), x[i].z, s0);
+            s1 = __builtin_fmaf(static_cast<float>(o[i].y), x[i].w, s1);
         }
         return s0 + s1;
     }
@@ -251,10 +244,12 @@ int wl_gemv_dtype(int type, const void* w, int64_t rows, int64_t k, int64_t row_
                      y_dtype == WL_DTYPE_BF16 ? 1 : 0, static_cast<hipStream_t>(stream)};
     if (x_dtype == WL_DTYPE_BF16) {
         const uint16_t* xb = static_cast<const uint16_t*>(x);
-        type == WL_TYPE_Q4_K ? launch_gemv<WL_TYPE_Q4_K>(g, xb, tokens, y) : launch_gemv<WL_TYPE_Q6_K>(g, xb, tokens, y);
+        type == WL_TYPE_Q4_K ? launch_gemv<WL_TYPE_Q4_K>(g, xb, tokens, y)
+                             : launch_gemv<WL_TYPE_Q6_K>(g, xb, tokens, y);
     } else {
         const float* xf = static_cast<const float*>(x);
-        type == WL_TYPE_Q4_K ? launch_gemv<WL_TYPE_Q4_K>(g, xf, tokens, y) : launch_gemv<WL_TYPE_Q6_K>(g, xf, tokens, y);
+        type == WL_TYPE_Q4_K ? launch_gemv<WL_TYPE_Q4_K>(g, xf, tokens, y)
+                             : launch_gemv<WL_TYPE_Q6_K>(g, xf, tokens, y);
     }
     return launch_status();
 }
