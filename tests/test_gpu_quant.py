@@ -135,6 +135,32 @@ def test_gemv_small_x(hip, name, rows, k, tokens):
     assert torch.equal(hip.gemv(raw, name, (rows, k), x * 2.0 ** -110), y * 2.0 ** -110)
 
 
+@pytest.mark.parametrize("name,rows,k", [
+    ("Q4_K", 33, 256), ("Q6_K", 37, 512), ("Q4_K", 130, 768), ("Q6_K", 31, 1024), ("Q4_K", 65, 1280), ("Q6_K", 70, 1792),
+    ("Q4_K", 4096, 2048), ("Q6_K", 2100, 2048), ("Q4_K", 4096, 2560), ("Q6_K", 1030, 4096), ("Q4_K", 8201, 2304),
+    ("Q6_K", 130, 8192), ("Q4_K", 2050, 8448), ("Q6_K", 17, 33024)])
+@pytest.mark.parametrize("tokens", [1, 3, 8])
+def test_gemv_sums_as_batch(hip, name, rows, k, tokens):
+    """gemv's bits are gemv_batch's for each token, whatever the split: blocks over lanes, over wavefronts (one round and
+    more, the last one short), 1, 2 and 4 rows per lane group, missing rows. fp32 in and out, and the two mixed forms:
+    bf16 x gives the bits of its fp32 values, bf16 y is y rounded once."""
+    rng = np.random.default_rng(rows + k + tokens)
+    raw = dev(synth.matrix(rng, name, rows, k)).reshape(-1)
+    xb = torch.from_numpy(rng.standard_normal((tokens, k)).astype(np.float32)).cuda().to(torch.bfloat16)
+    x = xb.float()
+    y = hip.gemv(raw, name, (rows, k), x)
+    alone = torch.zeros(1, rows, device="cuda")
+    for t in range(tokens):
+        hip.gemv_batch(raw, name, (rows, k), x[t], [0], [0], alone)
+        assert torch.equal(y[t], alone[0]), t
+    for xin, in_code, out_code, out in ((xb, hip.DTYPE_BF16, hip.DTYPE_F32, torch.empty_like(y)),
+                                        (x, hip.DTYPE_F32, hip.DTYPE_BF16, torch.empty_like(y, dtype=torch.bfloat16))):
+        assert hip.library().wl_gemv_dtype(hip.TYPE_IDS[name], raw.data_ptr(), rows, k, hip.row_bytes(name, k),
+                                           xin.data_ptr(), in_code, tokens, out.data_ptr(), out_code,
+                                           torch.cuda.current_stream().cuda_stream) == 0
+        assert torch.equal(out, y.to(out.dtype))
+
+
 def test_gemv_batch_and_combine(hip):
     """gate_up of 4 experts in one launch (gemv_batch), then down + weighted sum (gemv_combine), as
     Engine.batched_decode_experts drives them (engines/base.py:492-532)."""

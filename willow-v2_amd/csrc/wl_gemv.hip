@@ -82,36 +82,48 @@ __device__ __forceinline__ float pair_add16(float a, float b) {
            __builtin_bit_cast(float, static_cast<uint32_t>(r[1]));
 }
 
+// v[0 .. 3] each summed over the wavefront: row i of 16 lanes returns v[i]'s sum. Every level adds as group_sum<64>
+// does (addition commutes exactly), so the bits are its; the last two levels take one swap and one add for two values.
+__device__ __forceinline__ float quad_sum(const float (&v)[4]) {
+    float u[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) u[i] = group_sum<16>(v[i]);
+    return pair_add32(pair_add16(u[0], u[1]), pair_add16(u[2], u[3]));
+}
+
 // The matrix times TT tokens (1 .. 8). A block belongs to 8 lanes (wl_common.h), 2^ks blocks of a row to a wavefront
-// pass; a wavefront holds R rows in each of its 8 >> ks lane groups, and kw of the workgroup's 4 wavefronts split K
-// (their sums are added in LDS in a fixed order). The lane's x runs come straight from global memory (L2 and L1 hold
-// them) and serve R rows each.
-// What bounds it: at 8 tokens the products (8 FMAs per weight; Q6_K 2048 x 4096: 4,100 VALU cycles per SIMD = 1.7 us)
-// and the x reads, which are why a lane group holds several rows; at one token the launch and one trip to memory.
+// pass; a wavefront holds R rows in each of its 8 >> ks lane groups, and kw of the workgroup's 4 wavefronts split the
+// blocks of longer rows, 8 kw to a round. The lane's x runs come straight from global memory (L2 and L1 hold them) and
+// serve R rows each.
+// Every sum is added as k_gemv_batch adds it (wl_quant.hip): a lane its blocks slot, slot + 8, ... in order, then the
+// lanes, so a matrix gives the same bits alone and among batched experts, however its blocks are split. With kw > 1 a
+// round's products meet in LDS, lane by lane, and each wavefront adds up and reduces its share of the values. (Each
+// wavefront reducing its own products first, another order, took 10.8 us where this takes 11.8: Q4_K 4096 x 2560, 8
+// tokens.) LDS then: Q quads of values, [4][Q][64] products and [4 / kw][Q][64] running sums for more than one round.
+// What bounds it: at 8 tokens the x reads (a lane's 64-byte runs, 64 bytes apart) and the rows they are read for, which
+// is why a lane group holds several; at one token the launch and one trip to memory.
 // Measured per call in a graph (bf16 in and out; before: a row per wavefront, its x read again for every row, and a
-// converting launch on each side): Q4_K 4096 x 2048 at 1 token 8.2 -> 4.1 us, 8 tokens 21.5 -> 8.5; Q6_K 2048 x 4096
-// 9.3 -> 4.4 and 22.0 -> 8.7; Q4_K 2048 x 512 6.2 -> 2.9 and 10.1 -> 5.3.
+// converting launch on each side): Q4_K 4096 x 2048 at 1 token 8.4 -> 4.2 us, 8 tokens 21.9 -> 7.7; Q6_K 2048 x 4096
+// 9.7 -> 4.7 and 22.4 -> 8.9, 8 tokens of fp32 18.1 -> 9.0; Q4_K 2048 x 512 6.4 -> 3.0 and 10.4 -> 5.0.
 template <int TYPE, int TT, int R, typename XT>
 __global__ __launch_bounds__(256) void k_gemv(const uint8_t* __restrict__ w, int rows, int nb, int64_t row_stride,
                                               const XT* __restrict__ x, int64_t ldx, void* __restrict__ y,
                                               int64_t ldy, int y_bf16, int ks, int kw) {
-    constexpr int N = TT * R;
-    __shared__ float part[4][8 * N];  // [wavefront][(t R + r) subs + sub]
+    constexpr int N = TT * R;  // a lane's values: t R + r
+    extern __shared__ __attribute__((aligned(16))) float4 lds[];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int g = lane >> 3, c = lane & 7;
     const int slot = g & ((1 << ks) - 1), sub = g >> ks, subs = 8 >> ks;
     const int kwi = wv % kw, rset = wv / kw;
-    const int rows_wave = subs * R, rows_wg = 4 / kw * rows_wave;
-    const int wg_row0 = static_cast<int>(blockIdx.x) * rows_wg;
-    const int row0 = wg_row0 + rset * rows_wave + sub * R;
+    const int row0 = (static_cast<int>(blockIdx.x) * (4 / kw) + rset) * subs * R + sub * R;
     const int lo_start = BlockInfo<TYPE>::lo_start(c);
     const uint8_t* rp[R];
 #pragma unroll
     for (int r = 0; r < R; r++) rp[r] = w + static_cast<int64_t>(min(row0 + r, rows - 1)) * row_stride;
-    float acc[N];
+    float d[N];
 #pragma unroll
-    for (int n = 0; n < N; n++) acc[n] = 0.0f;
-    for (int kb = (kwi << ks) + slot; kb < nb; kb += kw << ks) {
+    for (int n = 0; n < N; n++) d[n] = 0.0f;
+    auto add_block = [&](int kb) {  // the lane's products of block kb
         RawLane<TYPE> raw[R];
 #pragma unroll
         for (int r = 0; r < R; r++) raw[r].fetch(rp[r] + static_cast<int64_t>(kb) * BlockInfo<TYPE>::bytes, c);
@@ -126,45 +138,81 @@ __global__ __launch_bounds__(256) void k_gemv(const uint8_t* __restrict__ w, int
             load_run16(xk + t * ldx + BlockInfo<TYPE>::hi_offset, xh);
             const float sxl = sum16(xl), sxh = sum16(xh);
 #pragma unroll
-            for (int r = 0; r < R; r++) acc[t * R + r] += h[r].run(xl, xh, sxl, sxh);
+            for (int r = 0; r < R; r++) d[t * R + r] += h[r].run(xl, xh, sxl, sxh);
         }
-    }
-    if (ks == 3) {
-        // over all 64 lanes: the first two steps halve the number of values, and row q of 16 lanes ends with value
-        // 4 i + (q >> 1) + 2 (q & 1) of quadruple i
-        float u[(N + 1) / 2], v[(N + 3) / 4];
-#pragma unroll
-        for (int i = 0; i < (N + 1) / 2; i++) u[i] = pair_add32(acc[2 * i], acc[2 * i + 1 < N ? 2 * i + 1 : 2 * i]);
-#pragma unroll
-        for (int i = 0; i < (N + 3) / 4; i++)
-            v[i] = group_sum<16>(pair_add16(u[2 * i], u[2 * i + 1 < (N + 1) / 2 ? 2 * i + 1 : 2 * i]));
-        const int q = lane >> 4, at = (q >> 1) + 2 * (q & 1);
-        if ((lane & 15) == 0) {
-#pragma unroll
-            for (int i = 0; i < (N + 3) / 4; i++)
-                if (4 * i + at < N) part[wv][4 * i + at] = v[i];
-        }
-    } else {
-#pragma unroll
-        for (int n = 0; n < N; n++) {
-            float s = group_sum<8>(acc[n]);
-            if (ks >= 1) s += dpp<0x140>(s);
-            if (ks >= 2) s = swap_add<16>(s);
-            if ((lane & ((8 << ks) - 1)) == 0) part[wv][n * subs + sub] = s;
-        }
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < TT * rows_wg; i += 256) {
-        const int t = i / rows_wg, rr = i - t * rows_wg, row = wg_row0 + rr;
-        if (row >= rows) continue;
-        const int rs = rr / rows_wave, in = rr - rs * rows_wave;
-        const int at = (t * R + in % R) * subs + in / R;
-        float s = part[rs * kw][at];
-        for (int j = 1; j < kw; j++) s += part[rs * kw + j][at];
+    };
+    auto store = [&](int n, float v) {
+        const int row = row0 + n % R;
+        if (row >= rows) return;
+        const int64_t at = (n / R) * ldy + row;
         if (y_bf16)
-            static_cast<uint16_t*>(y)[t * ldy + row] = static_cast<uint16_t>(f32_to_bf16_bits(s));
+            static_cast<uint16_t*>(y)[at] = static_cast<uint16_t>(f32_to_bf16_bits(v));
         else
-            static_cast<float*>(y)[t * ldy + row] = s;
+            static_cast<float*>(y)[at] = v;
+    };
+    if (kw == 1) {
+        if (slot < nb) add_block(slot);  // the only one up to 8 blocks a row
+        for (int kb = slot + 8; kb < nb; kb += 8) add_block(kb);
+        if (ks == 3) {
+#pragma unroll
+            for (int n = 0; n < N; n += 4) {
+                const float v[4] = {d[n], n + 1 < N ? d[n + 1] : 0.0f, n + 2 < N ? d[n + 2] : 0.0f,
+                                    n + 3 < N ? d[n + 3] : 0.0f};
+                const float s = quad_sum(v);
+                if ((lane & 15) == 0 && n + (lane >> 4) < N) store(n + (lane >> 4), s);
+            }
+        } else {
+#pragma unroll
+            for (int n = 0; n < N; n++) {
+                float s = group_sum<8>(d[n]);
+                if (ks >= 1) s += dpp<0x140>(s);
+                if (ks >= 2) s = swap_add<16>(s);
+                if ((lane & ((8 << ks) - 1)) == 0) store(n, s);
+            }
+        }
+        return;
+    }
+    // LDS holds quads of values, [wavefront][quad][lane] float4
+    constexpr int Q = (N + 3) / 4;
+    float4* mine = lds + wv * Q * 64 + lane;
+    const float4* part = lds + rset * kw * Q * 64 + lane;
+    float4* run = lds + (4 + rset) * Q * 64 + lane;
+    if (8 * kwi + slot < nb) add_block(8 * kwi + slot);  // the first round, the only one up to 8 kw blocks a row
+    for (int kb0 = 8 * kw;; kb0 += 8 * kw) {
+#pragma unroll
+        for (int i = 0; i < Q; i++)
+            mine[i * 64] = make_float4(d[4 * i], 4 * i + 1 < N ? d[4 * i + 1] : 0.0f,
+                                       4 * i + 2 < N ? d[4 * i + 2] : 0.0f, 4 * i + 3 < N ? d[4 * i + 3] : 0.0f);
+        __syncthreads();
+        const bool last = kb0 >= nb;
+        for (int i = kwi; i < Q; i += kw) {
+            float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (kb0 > 8 * kw) s = run[i * 64];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                if (j < kw) {
+                    const float4 p = part[(j * Q + i) * 64];
+                    s.x += p.x;
+                    s.y += p.y;
+                    s.z += p.z;
+                    s.w += p.w;
+                }
+            }
+            if (last) {
+                const float v[4] = {s.x, s.y, s.z, s.w};
+                const float sum = quad_sum(v);
+                const int n = 4 * i + (lane >> 4);
+                if ((lane & 15) == 0 && n < N) store(n, sum);
+            } else {
+                run[i * 64] = s;
+            }
+        }
+        if (last) return;
+#pragma unroll
+        for (int n = 0; n < N; n++) d[n] = 0.0f;
+        const int kb = kb0 + 8 * kwi + slot;
+        if (kb < nb) add_block(kb);
+        __syncthreads();  // the round's products are read
     }
 }
 
@@ -184,21 +232,29 @@ template <int TYPE, int TT, int R, typename XT>
 static void launch_gemv_r(const GemvCall& g, const XT* x, void* y, int ks, int kw) {
     const int rows_wg = 4 / kw * (8 >> ks) * R;
     const unsigned grid = static_cast<unsigned>((g.rows + rows_wg - 1) / rows_wg);
-    k_gemv<TYPE, TT, R, XT><<<grid, 256, 0, g.s>>>(g.w, g.rows, g.nb, g.row_stride, x, g.k, y, g.rows, g.y_bf16, ks,
+    constexpr int Q = (TT * R + 3) / 4;
+    const size_t lds = kw == 1 ? 0 : static_cast<size_t>(4 + (g.nb > 8 * kw ? 4 / kw : 0)) * Q * 64 * sizeof(float4);
+    k_gemv<TYPE, TT, R, XT><<<grid, 256, lds, g.s>>>(g.w, g.rows, g.nb, g.row_stride, x, g.k, y, g.rows, g.y_bf16, ks,
                                                    kw);
 }
 
 template <int TYPE, int TT, typename XT>
 static void launch_gemv_t(const GemvCall& g, const XT* x, void* y) {
-    const int ks = g.nb >= 8 ? 3 : g.nb >= 4 ? 2 : g.nb >= 2 ? 1 : 0;
-    const int kw = g.nb <= 8 ? 1 : g.nb <= 16 ? 2 : 4;
+    const int ks = g.nb > 4 ? 3 : g.nb > 2 ? 2 : g.nb > 1 ? 1 : 0;
+    // wavefronts per row: up to 16 blocks one wavefront's two passes do where the rows alone are enough workgroups (us
+    // with 1 / 2; 8 tokens of fp32, Q4_K 8192 x 4096 20.8 / 23.6, 4096 x 2560 12.6 / 11.9)
+    const int kw = g.nb <= 8 || (g.nb <= 16 && g.rows >= 8192) ? 1 : g.nb <= 16 ? 2 : 4;
     const int per_r = 4 / kw * (8 >> ks);  // rows of a workgroup per R
-    // rows per lane group: more reuse each x read, fewer leave more workgroups. From 512 workgroups on (1024 for one
-    // token, whose x reads are few) more rows win (us with 1 / 2 / 4 rows; Q6_K 8192 x 2048, 8 tokens 17.5 / 15.0 /
-    // 13.0, 1 token 7.0 / 6.4 / 7.0; Q6_K 2048 x 4096, 8 tokens 10.3 / 8.7 / 9.3); with fewer the launch is too thin
-    // (Q4_K 1024 x 2048, 8 tokens 5.6 / 6.4 / 7.8)
-    const int64_t least = TT == 1 ? 1024 : 512;
-    const int want = g.rows >= 4 * per_r * least ? 4 : g.rows >= 2 * per_r * least ? 2 : 1;
+    // rows per lane group: more reuse each x read, fewer leave more workgroups. Two from 256 workgroups on (us with 1 /
+    // 2 / 4 rows; 8 tokens of bf16, Q4_K 2048 x 2048 6.6 / 5.5 / 7.2, 1024 x 2048 4.8 / 5.4 / 7.1). Four from 256 on
+    // where x is read most (8 tokens of fp32, Q4_K 4096 x 2048 17.1 / 10.7 / 8.3; bf16, 2048 x 4096 11.1 / 9.2 / 8.6),
+    // else from 512 (bf16, 2 tokens, 4096 x 2048 5.0 / 4.5 / 4.9; 8 tokens, 8192 x 2048 18.7 / 14.8 / 11.5), and for
+    // one token of bf16 from 1024 (8192 x 2048 6.1 / 5.1 / 5.3, 151936 x 2048 71 / 55 / 46). One token and Q6_K
+    // never: its raw blocks fill the registers (8192 x 4096 9.2 / 8.5 / 9.1).
+    constexpr bool kBf16 = sizeof(XT) == 2;
+    const int64_t least4 = TT == 1 ? (kBf16 ? 1024 : 512) : TT == 2 || (kBf16 && kw != 2) ? 512 : 256;
+    const bool four = !(TT == 1 && TYPE == WL_TYPE_Q6_K) && g.rows >= 4 * per_r * least4;
+    const int want = four ? 4 : g.rows >= 2 * per_r * 256 ? 2 : 1;
     if (want == 4)
         launch_gemv_r<TYPE, TT, 4>(g, x, y, ks, kw);
     else if (want == 2)
