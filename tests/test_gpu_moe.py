@@ -496,3 +496,16 @@ def test_pre_norm_in_router(hip, hidden, T, weighted):
     np.testing.assert_array_equal(ids, ids_plain)
     np.testing.assert_array_equal(wts.view(np.uint32), wts_plain.view(np.uint32))
     np.testing.assert_array_equal(y.view(np.uint32), (x + y_plain).view(np.uint32))
+
+
+@pytest.mark.parametrize("T", [48, 49])
+def test_pre_norm_rule_edge(hip, c2, layer_c2, c2_norm_weight, T):
+    """Both sides of the rule that puts the normalization in the router's launch or before it (256 experts: 204 and 272
+    workgroups), bit for bit the plain layer on the oracle's rms_norm(x)."""
+    layer = hip.MoELayer.from_host(layer_c2, pre_norm=True, norm_weight=c2_norm_weight, norm_eps=1e-6)
+    x = synth.tokens(6, T) * np.float32(3.0)
+    y, ids, wts = run_layer(hip, layer, x)
+    y_plain, ids_plain, wts_plain = run_layer(hip, c2, moe_ref.rms_norm(x, c2_norm_weight, 1e-6))
+    np.testing.assert_array_equal(ids, ids_plain)
+    np.testing.assert_array_equal(wts.view(np.uint32), wts_plain.view(np.uint32))
+    np.testing.assert_array_equal(y.view(np.uint32), y_plain.view(np.uint32))

@@ -201,7 +201,8 @@ __global__ __launch_bounds__(256) void k_topk(const float* __restrict__ logits, 
 // of its 16 tokens (k_rms_norm's order, so the same bits), each token's row read once, contiguously, and cut into
 // segments through the wavefront's staging area; the first row tile's workgroups store the normalized values for the
 // expert kernels. As a launch of its own the norm took 7.7 us of a 5-token layer (its lanes read 256 bytes apart, 64
-// lines a load; the same reads in here saved nothing): layer 67.9 -> 63.6 us at 5 tokens, 47 -> 42.8 at 2.
+// lines a load; the same reads in here saved nothing): layer 67.3 -> 63.0 us at 5 tokens, 47 -> 42.8 at 2. Every
+// workgroup reads its tokens' whole rows for it, so many workgroups cost more than the launch (norm_in_router).
 struct NormIn {
     const float* w;  // nullable
     float eps;
@@ -1396,6 +1397,25 @@ static size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 // Whether wl_moe_layer's router runs as k_router_parts + k_topk_parts (a single token runs the fused kernel).
 static bool router_parts(int64_t T) { return T >= 2 && T <= kRouterPartsMaxT; }
 
+static dim3 router_parts_grid(const WlMoeLayer& L, int64_t T) {
+    const int rows = L.n_experts + ((L.shared_gate_up && L.shared_gate) ? 1 : 0);
+    const int nseg = L.hidden / kRouterSeg;
+    return dim3(static_cast<unsigned>((T + 15) / 16), static_cast<unsigned>((rows + 15) / 16),
+                static_cast<unsigned>((nseg + kRsWaves - 1) / kRsWaves));
+}
+
+// Whether k_router_parts also normalizes a pre-norm call's rows: while a CU has at most two rows' sums of squares to
+// take one after another, counting a wavefront's rows (two from 9 tokens on) times the rounds of workgroups (82 KiB of
+// LDS, one to a CU). Layer us as its own launch / in the router: hidden 2048, 256 experts, 48 tokens (204 workgroups) 207 /
+// 207, 56 (272) 215 / 222; hidden 4096, 512 experts, 8 tokens (264) 96 / 81, 16 tokens (264) 118 / 122, 48 tokens (792)
+// 184 / 219.
+static bool norm_in_router(const WlMoeLayer& L, int64_t T) {
+    if (!router_parts(T)) return false;
+    const dim3 g = router_parts_grid(L, T);
+    const unsigned rounds = (g.x * g.y * g.z + 255) / 256;
+    return rounds * (T > kRsWaves ? 2 : 1) <= 2;
+}
+
 Workspace carve(const WlMoeLayer& L, int64_t T, void* base) {
     Workspace w{};
     const int64_t P = T * L.top_k;
@@ -1520,12 +1540,8 @@ static int launch_topk(const WlMoeLayer& L, const float* logits, int64_t T, int3
 static int launch_router_parts(const WlMoeLayer& L, const float* x, int64_t T, const Workspace& w, uint16_t* xb,
                                bool norm, hipStream_t s) {
     const float* shared_gate = (L.shared_gate_up && L.shared_gate) ? L.shared_gate : nullptr;
-    const int rows = L.n_experts + (shared_gate ? 1 : 0);
-    const int nseg = L.hidden / kRouterSeg;
     auto kernel = norm ? k_router_parts<true> : k_router_parts<false>;
-    const dim3 grid(static_cast<unsigned>((T + 15) / 16), static_cast<unsigned>((rows + 15) / 16),
-                    static_cast<unsigned>((nseg + kRsWaves - 1) / kRsWaves));
-    kernel<<<grid, 64 * kRsWaves, 0, s>>>(x, L.router, shared_gate, static_cast<int>(T), L.hidden, L.n_experts, w.parts,
+    kernel<<<router_parts_grid(L, T), 64 * kRsWaves, 0, s>>>(x, L.router, shared_gate, static_cast<int>(T), L.hidden, L.n_experts, w.parts,
                                           xb, w.sync + kTopkDone, NormIn{L.norm_weight, L.norm_eps, w.xn});
     return launch_status();
 }
@@ -1854,10 +1870,10 @@ static int run_layer(const WlMoeLayer* layer, const float* x, int64_t tokens, fl
     auto mark = record;
     mark(0);
     const float* resid = (L.flags & WL_MOE_RESIDUAL) ? x : nullptr;
-    // every stage below runs on the normalized input; up to kRouterPartsMaxT tokens the router makes it
+    // every stage below runs on the normalized input, which the router makes where norm_in_router says so
     const float* router_x = x;
-    const bool norm_in_router = (L.flags & WL_MOE_PRE_NORM) && router_parts(tokens);
-    if (norm_in_router) {
+    const bool router_norm = (L.flags & WL_MOE_PRE_NORM) && norm_in_router(L, tokens);
+    if (router_norm) {
         x = w.xn;
     } else if (L.flags & WL_MOE_PRE_NORM) {
         k_rms_norm<<<static_cast<unsigned>((tokens + 3) / 4), 256, 0, s>>>(x, L.norm_weight, L.norm_eps,
@@ -1888,7 +1904,7 @@ static int run_layer(const WlMoeLayer* layer, const float* x, int64_t tokens, fl
     }
     const bool starve = (L.flags & WL_MOE_TEST_STARVE) != 0;
     if (router_parts(tokens)) {
-        rc = launch_router_parts(L, router_x, tokens, w, mfma ? w.xb : nullptr, norm_in_router, s);
+        rc = launch_router_parts(L, router_norm ? router_x : x, tokens, w, mfma ? w.xb : nullptr, router_norm, s);
         if (rc) return rc;
         mark(1);
         // the grouping in the same launch (mark 3 follows mark 2 at once)
