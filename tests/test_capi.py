@@ -70,6 +70,19 @@ def test_gemv_null_and_dtype():
     assert lib.wl_dequant(12, FAKE, 4, 256, 144, 7, FAKE, None) == -7
 
 
+@pytest.mark.parametrize("args,code", [
+    ((3, 12, FAKE, 4, 256, 144, FAKE, 1, FAKE, 0), -7), ((0, 12, FAKE, 4, 256, 144, FAKE, 1, FAKE, -1), -7),
+    ((1, 12, FAKE, 4, 256, 144, FAKE + 2, 1, FAKE, 1), -4), ((1, 12, FAKE, 4, 256, 144, FAKE + 8, 1, FAKE, 0), -4),
+    ((1, 12, FAKE, 4, 256, 144, None, 1, FAKE, 1), -3), ((0, 12, FAKE, 4, 256, 144, FAKE, 1, None, 1), -3),
+    ((1, 12, FAKE, 4, 256, 144, FAKE, 0, FAKE, 1), -2), ((1, 12, FAKE, 4, 256, 128, FAKE, 1, FAKE, 1), -2),
+    ((1, 14, FAKE, 4, 256, 211, FAKE, 1, FAKE, 1), -4), ((1, 13, FAKE, 4, 256, 176, FAKE, 1, FAKE, 1), -1)])
+def test_gemv_dtype_validation(args, code):
+    """wl_gemv_dtype refuses what wl_gemv does, and unknown dtype codes of x (first) and y (last)."""
+    x_dtype, type_id, w, rows, k, stride, x, tokens, y, y_dtype = args
+    lib = hip.library()
+    assert lib.wl_gemv_dtype(type_id, w, rows, k, stride, x, x_dtype, tokens, y, y_dtype, None) == code
+
+
 def test_batch_validation():
     lib = hip.library()
     offs = hip._int64_array([0, 144 * 4])

@@ -359,6 +359,26 @@ def test_prefill_small_tiles(hip, gate_up, down, inter, T):
     check_prefill(hip, hip.MoELayer.from_host(lw, mfma="always"), lw, synth.tokens(73, T, 1024), f"small tiles {T}")
 
 
+@pytest.mark.parametrize("gate_up,down,inter,T", [("Q4_K", "Q6_K", 1024, 150), ("Q6_K", "Q4_K", 1024, 200),
+                                                    ("Q4_K", "Q4_K", 1280, 280), ("Q6_K", "Q6_K", 768, 300)])
+def test_prefill_large_tiles(hip, gate_up, down, inter, T):
+    """More than 64 tokens per expert: the 144- and 128-token tiles with 3 to 5 blocks a down row (double-buffered, and in
+    phases for short last tiles) give, bit for bit, what the 64-token tiles give for the same tokens in smaller calls,
+    which test_prefill_small_tiles holds against the oracle: the same products in the same order. (Against the oracle
+    itself the largest difference over this many outputs is one bf16 rounding that falls the other way at an output near
+    the largest, up to 2^-7 of it.)"""
+    lw = synth.moe_layer(76, hidden=1280, inter=inter, shared_inter=inter, experts=8, top_k=4, gate_up_type=gate_up,
+                         down_type=down)
+    layer = hip.MoELayer.from_host(lw, mfma="always")
+    x = synth.tokens(77, T, 1280)
+    y, ids, wts = run_layer(hip, layer, x)
+    parts = [run_layer(hip, layer, xc) for xc in np.array_split(x, (T + 99) // 100)]  # of 66 to 100 tokens
+    np.testing.assert_array_equal(ids, np.concatenate([p[1] for p in parts]))
+    np.testing.assert_array_equal(wts.view(np.uint32), np.concatenate([p[2] for p in parts]).view(np.uint32))
+    np.testing.assert_array_equal(y.view(np.uint32), np.concatenate([p[0] for p in parts]).view(np.uint32))
+    assert moe_ref.rel_err(y, moe_ref.layer(x, lw)) < 2e-2
+
+
 @pytest.mark.parametrize("T", [12, 64])
 def test_mfma_small_batches_k_split(hip, layer_c2, T):
     """At most 64 tokens with every expert on the MFMA GEMMs (the full-shape layer): the K-split kernels, gate_up's
