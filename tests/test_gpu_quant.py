@@ -269,12 +269,30 @@ def test_linear_mfma(hip, name, rows, k, tokens):
 @pytest.mark.parametrize("name,rows,k,tokens", [
     ("Q4_K", 256, 768, 9), ("Q6_K", 768, 1280, 65), ("Q4_K", 2304, 2048, 200), ("Q6_K", 256, 1024, 449),  # K 4 ways
     ("Q6_K", 512, 512, 17), ("Q4_K", 768, 512, 500), ("Q6_K", 2048, 1280, 700),                           # K 2 ways
-    ("Q4_K", 4096, 256, 130), ("Q6_K", 4096, 1280, 1000), ("Q4_K", 4096, 768, 640),                   # 64-token tiles
-    ("Q6_K", 4096, 512, 1300)])                                                                      # 128-token tiles
+    ("Q4_K", 4096, 256, 130), ("Q4_K", 4096, 768, 640),                                               # 64-token tiles
+    ("Q6_K", 4096, 1280, 1000), ("Q6_K", 4096, 512, 1300)])                                          # 128-token tiles
 def test_linear_mfma_forms(hip, name, rows, k, tokens):
     """Each kernel of wl_linear at its edges: block counts that do not divide into the K split, fewer than 8 token
     tiles and 8 or more, row slabs that do not fill the 8 XCDs, a last tile of 1, 8, 17 and 64 tokens. Bound: bf16's
     half ulp on the output (up to 2^-8 of its value) plus the fp32 sums' rounding (k 2^-24 of sum |w x|)."""
+    rng = np.random.default_rng(rows + k + tokens)
+    w = synth.matrix(rng, name, rows, k)
+    x = rng.standard_normal((tokens, k)).astype(np.float32)
+    y = hip.linear_mfma(dev(w).reshape(-1), name, (rows, k), torch.from_numpy(x).cuda()).float().cpu().numpy()
+    wb = q.round_bf16(q.dequantize_matrix(w, name, rows, k)).astype(np.float64)
+    xb = q.round_bf16(x).astype(np.float64)
+    ref, size = xb @ wb.T, np.abs(xb) @ np.abs(wb).T
+    assert (np.abs(y - ref) <= 2.0 ** -8 * np.abs(ref) + k * 2.0 ** -24 * size).all()
+
+
+@pytest.mark.parametrize("name,rows,k,tokens", [
+    ("Q6_K", 4096, 1536, 1000), ("Q6_K", 1280, 768, 700),           # 64-token tiles, an even and an odd number of blocks
+    ("Q4_K", 4096, 2048, 1290), ("Q6_K", 4096, 2048, 1300), ("Q4_K", 2048, 1280, 2900), ("Q6_K", 4096, 2304, 1370),
+    ("Q4_K", 8192, 1024, 570), ("Q6_K", 3072, 256, 1100), ("Q6_K", 16384, 768, 400), ("Q4_K", 16384, 1280, 390)])
+def test_linear_mfma_large_tiles(hip, name, rows, k, tokens):
+    """wl_linear's 128-token tiles (but for the first two), with 1 to 9 blocks a row: double-buffered, and in phases for a
+    last tile of 10 to 64 tokens (10, 20, 84, 90, 58, 76, 16, 6); 8 tiles and more, and fewer (dealt by row slabs). The
+    bound is test_linear_mfma_forms'."""
     rng = np.random.default_rng(rows + k + tokens)
     w = synth.matrix(rng, name, rows, k)
     x = rng.standard_normal((tokens, k)).astype(np.float32)

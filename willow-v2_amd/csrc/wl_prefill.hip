@@ -1315,14 +1315,20 @@ int launch_mfma_down(const WlMoeLayer& L, int64_t T, const Workspace& w, int gem
     return launch_status();
 }
 
-// The kernel of a wl_linear call, by how many workgroups it would run. While one round of the CUs takes them (a K-split
-// workgroup fills one), the K loop split 4 ways, or 2 with up to two blocks a row, is the shortest chain; then 64-token
-// tiles, three workgroups a CU; then the 128-token tiles, which decode each weight half as often. us by kernel, and
-// before (128-token tiles always): Q4_K 4096 x 2048, 200 tokens, 4 ways 12.5, 64-token tiles 24.5, before 38.5; 500
-// tokens 4 ways 25.3 (two rounds), 2 ways 20.8, 64-token 25.1, before 39.2; 1000 tokens 2 ways 37.6, 64-token 28.6,
-// before 40.8; 2048 tokens (1024 workgroups) 64-token 57.1, 128-token 44.3. Q6_K 4096 x 512, 1500 tokens (768) 20.8
-// and 20.7.
-constexpr int64_t kLinearKsGroups = 256, kLinearSmallGroups = 640;
+// The kernel of a wl_linear call, by the workgroups its grid would hold (with the padding of linear_grid: the token
+// tiles of one XCD are what it waits for). While one round of the CUs takes them (a K-split workgroup fills one),
+// the K loop split 4 ways, or 2 with up to two blocks a row, is the shortest chain; then 64-token tiles, three
+// workgroups a CU; then the 128-token tiles, which decode each weight half as often. us by kernel, K split 4 / 2
+// ways, 64-, 128-token tiles: Q4_K 4096 x 2048, 200 tokens 12.5 / - / 24.5 / 38.5, 500 tokens 25.3 / 20.8 / 25.1 /
+// 39.2, 1000 tokens (512 workgroups of 64-token tiles) - / 37.6 / 28.6 / 40.8, 2048 tokens (1024) - / - / 57.1 /
+// 44.3. The decode of Q6_K costs more: two workgroups of 64-token tiles on a CU share its VALU and three lose: 2048
+// x 4096, 2000 tokens (512) 112.9 / 109.8 / 82.7 / 95.0, 2500 (640) 140 / 162 / 110 / 95.5. Rows of an odd number
+// of Q6_K blocks, every other one off a dword boundary, make the wide loads slower, so there one a CU: 1280 x 768,
+// 64- / 128-token tiles, 700 tokens (160) 18.1 / 23.0, 2000 tokens (320) 25.9 / 23.8.
+constexpr int64_t kLinearKsGroups = 256;
+static int64_t linear_small_groups(int type, int blocks) {
+    return type == WL_TYPE_Q4_K ? 640 : blocks % 2 == 0 ? 512 : 256;
+}
 
 // y[t, :] = W x[t, :] for a single quantized matrix on the down GEMM: bf16 operands (x as given, W's exact values
 // rounded to bf16 in registers), fp32 accumulation, bf16 output. rows and k are multiples of 256.
@@ -1340,9 +1346,8 @@ int launch_linear(int type, const uint8_t* w, int rows, int k, const uint16_t* x
     a.down_slabs = 1;
     a.dense_tokens = static_cast<int>(T);
     const bool q4 = type == WL_TYPE_Q4_K;
-    const int64_t tiles = (T + kSmallTileTokens - 1) / kSmallTileTokens;
     static_assert(kKsTile == kSmallTileTokens, "");
-    auto groups = [&](int wg_rows) { return tiles * (rows / wg_rows); };
+    auto groups = [&](int wg_rows) -> int64_t { return linear_grid(rows / wg_rows, T, kSmallTileTokens); };
     auto grid = [&](int wg_rows, int cap) { return dim3(linear_grid(rows / wg_rows, T, cap)); };
     if (k > 2 * kQK && groups(ks_rows<4>()) <= kLinearKsGroups)
         (q4 ? k_gemm_down_ks<WL_TYPE_Q4_K, 4> : k_gemm_down_ks<WL_TYPE_Q6_K, 4>)
@@ -1350,7 +1355,7 @@ int launch_linear(int type, const uint8_t* w, int rows, int k, const uint16_t* x
     else if (k > kQK && groups(ks_rows<2>()) <= kLinearKsGroups)
         (q4 ? k_gemm_down_ks<WL_TYPE_Q4_K, 2> : k_gemm_down_ks<WL_TYPE_Q6_K, 2>)
             <<<grid(ks_rows<2>(), kKsTile), kGemmThreads, 0, s>>>(a);
-    else if (groups(gemm_rows<kSmallTileTokens>()) <= kLinearSmallGroups)
+    else if (groups(gemm_rows<kSmallTileTokens>()) <= linear_small_groups(type, k / kQK))
         (q4 ? k_gemm_down<WL_TYPE_Q4_K, kSmallTileTokens> : k_gemm_down<WL_TYPE_Q6_K, kSmallTileTokens>)
             <<<grid(gemm_rows<kSmallTileTokens>(), kSmallTileTokens), 64 * kSmallWaves, 0, s>>>(a);
     else
