@@ -791,7 +791,9 @@ __device__ __forceinline__ void gemm_tile(uint8_t (&bufs)[gemm_lds<TILE>()], flo
             gemm_loop_tiny<TYPE, 4, NTA>(bufs, acc, nblocks, nitems, s8, rowtab, row_ptr, epi, lr, q);
         else if (count > 32)
             gemm_loop_tiny<TYPE, 3, NTA>(bufs, acc, nblocks, nitems, s8, rowtab, row_ptr, epi, lr, q);
-        else if (count > 16)
+        // one token tile of Q6_K rows runs as two: the loop of its own spilled 7 of k_gemm_down's 168 registers (500
+        // tokens, layer 269.6 -> 263.2 us without it, 300 tokens 315.9 -> 312.4)
+        else if (count > 16 || TYPE == WL_TYPE_Q6_K)
             gemm_loop_tiny<TYPE, 2, NTA>(bufs, acc, nblocks, nitems, s8, rowtab, row_ptr, epi, lr, q);
         else
             gemm_loop_tiny<TYPE, 1, NTA>(bufs, acc, nblocks, nitems, s8, rowtab, row_ptr, epi, lr, q);
