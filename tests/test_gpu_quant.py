@@ -139,7 +139,8 @@ def test_gemv_small_x(hip, name, rows, k, tokens):
 @pytest.mark.parametrize("name,rows,k", [
     ("Q4_K", 33, 256), ("Q6_K", 37, 512), ("Q4_K", 130, 768), ("Q6_K", 31, 1024), ("Q4_K", 65, 1280), ("Q6_K", 70, 1792),
     ("Q4_K", 4096, 2048), ("Q6_K", 2100, 2048), ("Q4_K", 4096, 2560), ("Q6_K", 1030, 4096), ("Q4_K", 8201, 2304),
-    ("Q6_K", 130, 8192), ("Q4_K", 2050, 8448), ("Q6_K", 17, 33024)])
+    ("Q6_K", 700, 2816), ("Q6_K", 600, 4352), ("Q6_K", 130, 8192), ("Q4_K", 2050, 8448), ("Q4_K", 300, 8704),
+    ("Q6_K", 17, 33024)])
 @pytest.mark.parametrize("tokens", [1, 3, 8])
 def test_gemv_sums_as_batch(hip, name, rows, k, tokens):
     """gemv's bits are gemv_batch's for each token, whatever the split: blocks over lanes, over wavefronts (one round and

@@ -91,27 +91,31 @@ __device__ __forceinline__ float quad_sum(const float (&v)[4]) {
     return pair_add32(pair_add16(u[0], u[1]), pair_add16(u[2], u[3]));
 }
 
-// The matrix times TT tokens (1 .. 8). A block belongs to 8 lanes (wl_common.h), 2^ks blocks of a row to a wavefront
-// pass; a wavefront holds R rows in each of its 8 >> ks lane groups, and kw of the workgroup's 4 wavefronts split the
-// blocks of longer rows, 8 kw to a round. The lane's x runs come straight from global memory (L2 and L1 hold them) and
-// serve R rows each.
-// Every sum is added as k_gemv_batch adds it (wl_quant.hip): a lane its blocks slot, slot + 8, ... in order, then the
-// lanes, so a matrix gives the same bits alone and among batched experts, however its blocks are split. With kw > 1 a
-// round's products meet in LDS, lane by lane, and each wavefront adds up and reduces its share of the values. (Each
-// wavefront reducing its own products first, another order, took 10.8 us where this takes 11.8: Q4_K 4096 x 2560, 8
-// tokens.) LDS then: Q quads of values, [4][Q][64] products and [4 / kw][Q][64] running sums for more than one round.
-// What bounds it: at 8 tokens the x reads (a lane's 64-byte runs, 64 bytes apart) and the rows they are read for, which
-// is why a lane group holds several; at one token the launch and one trip to memory.
+// The matrix times TT tokens (1 .. 8). A block belongs to 8 lanes (wl_common.h), 2^ks blocks of a row to a
+// wavefront pass; a wavefront holds R rows in each of its 8 >> ks lane groups, and kw of the workgroup's 4
+// wavefronts split the blocks of longer rows, 8 kw to a round (MORE: more than one round, more than 32 blocks a
+// row; apart, because its loop costs every shorter row registers). The lane's x runs come straight from global
+// memory (L2 and L1 hold them) and serve R rows each.
+// Every sum is added as k_gemv_batch adds it (wl_quant.hip): a lane its blocks slot, slot + 8, ... in order, then
+// the lanes, so a matrix gives the same bits alone and among batched experts, however its blocks are split. With kw
+// > 1 a round's products meet in LDS, lane by lane, in quads of values, Q of them, and each wavefront adds up and
+// reduces its share: with kw = 2 a wavefront hands over the quads that it does not finish itself ([2][Q][64] of
+// LDS), with kw = 4 all of them ([4][Q][64], and [Q][64] running sums when MORE). Both that way with kw = 2 took
+// 12.0 us where this takes 10.9, as sums reduced before they meet, in another order, did (Q4_K 4096 x 2560, 8
+// tokens of bf16).
+// What bounds it: at 8 tokens the x reads (a lane's 64-byte runs, 64 bytes apart) and the rows they are read for,
+// which is why a lane group holds several; at one token the launch and one trip to memory.
 // Measured per call in a graph (bf16 in and out; before: a row per wavefront, its x read again for every row, and a
-// converting launch on each side): Q4_K 4096 x 2048 at 1 token 8.4 -> 4.2 us, 8 tokens 21.9 -> 7.7; Q6_K 2048 x 4096
-// 9.7 -> 4.7 and 22.4 -> 8.9, 8 tokens of fp32 18.1 -> 9.0; Q4_K 2048 x 512 6.4 -> 3.0 and 10.4 -> 5.0.
-template <int TYPE, int TT, int R, typename XT>
+// converting launch on each side): Q4_K 4096 x 2048 at 1 token 8.5 -> 4.2 us, 8 tokens 21.8 -> 7.6; Q6_K 2048 x
+// 4096 9.6 -> 4.4 and 22.2 -> 8.2, 8 tokens of fp32 18.1 -> 8.5; Q4_K 2048 x 512 6.5 -> 3.0 and 10.6 -> 5.1.
+template <int TYPE, int TT, int R, typename XT, bool MORE>
 __global__ __launch_bounds__(256) void k_gemv(const uint8_t* __restrict__ w, int rows, int nb, int64_t row_stride,
                                               const XT* __restrict__ x, int64_t ldx, void* __restrict__ y,
                                               int64_t ldy, int y_bf16, int ks, int kw) {
-    constexpr int N = TT * R;  // a lane's values: t R + r
+    constexpr int N = TT * R, Q = (N + 3) / 4;  // a lane's values, t R + r, and quads of them
     extern __shared__ __attribute__((aligned(16))) float4 lds[];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
     const int g = lane >> 3, c = lane & 7;
     const int slot = g & ((1 << ks) - 1), sub = g >> ks, subs = 8 >> ks;
     const int kwi = wv % kw, rset = wv / kw;
@@ -150,17 +154,21 @@ __global__ __launch_bounds__(256) void k_gemv(const uint8_t* __restrict__ w, int
         else
             static_cast<float*>(y)[at] = v;
     };
+    auto quad = [&](int i) {
+        return make_float4(d[4 * i], 4 * i + 1 < N ? d[4 * i + 1] : 0.0f, 4 * i + 2 < N ? d[4 * i + 2] : 0.0f,
+                           4 * i + 3 < N ? d[4 * i + 3] : 0.0f);
+    };
+    auto finish = [&](int i, const float4& s) {  // quad i's lanes added and stored
+        const float v[4] = {s.x, s.y, s.z, s.w};
+        const float sum = quad_sum(v);
+        const int n = 4 * i + (lane >> 4);
+        if ((lane & 15) == 0 && n < N) store(n, sum);
+    };
+    if (8 * kwi + slot < nb) add_block(8 * kwi + slot);
     if (kw == 1) {
-        if (slot < nb) add_block(slot);  // the only one up to 8 blocks a row
-        for (int kb = slot + 8; kb < nb; kb += 8) add_block(kb);
         if (ks == 3) {
 #pragma unroll
-            for (int n = 0; n < N; n += 4) {
-                const float v[4] = {d[n], n + 1 < N ? d[n + 1] : 0.0f, n + 2 < N ? d[n + 2] : 0.0f,
-                                    n + 3 < N ? d[n + 3] : 0.0f};
-                const float s = quad_sum(v);
-                if ((lane & 15) == 0 && n + (lane >> 4) < N) store(n + (lane >> 4), s);
-            }
+            for (int i = 0; i < Q; i++) finish(i, quad(i));
         } else {
 #pragma unroll
             for (int n = 0; n < N; n++) {
@@ -170,49 +178,57 @@ __global__ __launch_bounds__(256) void k_gemv(const uint8_t* __restrict__ w, int
                 if ((lane & ((8 << ks) - 1)) == 0) store(n, s);
             }
         }
-        return;
-    }
-    // LDS holds quads of values, [wavefront][quad][lane] float4
-    constexpr int Q = (N + 3) / 4;
-    float4* mine = lds + wv * Q * 64 + lane;
-    const float4* part = lds + rset * kw * Q * 64 + lane;
-    float4* run = lds + (4 + rset) * Q * 64 + lane;
-    if (8 * kwi + slot < nb) add_block(8 * kwi + slot);  // the first round, the only one up to 8 kw blocks a row
-    for (int kb0 = 8 * kw;; kb0 += 8 * kw) {
+    } else if (kw == 2) {
+        constexpr int Q0 = (Q + 1) / 2;  // wavefront 0 finishes quads 0 .. Q0 - 1
+        float4* area = lds + rset * Q * 64 + lane;
+        if (kwi == 0) {
 #pragma unroll
-        for (int i = 0; i < Q; i++)
-            mine[i * 64] = make_float4(d[4 * i], 4 * i + 1 < N ? d[4 * i + 1] : 0.0f,
-                                       4 * i + 2 < N ? d[4 * i + 2] : 0.0f, 4 * i + 3 < N ? d[4 * i + 3] : 0.0f);
-        __syncthreads();
-        const bool last = kb0 >= nb;
-        for (int i = kwi; i < Q; i += kw) {
-            float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            if (kb0 > 8 * kw) s = run[i * 64];
+            for (int i = Q0; i < Q; i++) area[i * 64] = quad(i);
+        } else {
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                if (j < kw) {
-                    const float4 p = part[(j * Q + i) * 64];
-                    s.x += p.x;
-                    s.y += p.y;
-                    s.z += p.z;
-                    s.w += p.w;
-                }
-            }
-            if (last) {
-                const float v[4] = {s.x, s.y, s.z, s.w};
-                const float sum = quad_sum(v);
-                const int n = 4 * i + (lane >> 4);
-                if ((lane & 15) == 0 && n < N) store(n, sum);
-            } else {
-                run[i * 64] = s;
-            }
+            for (int i = 0; i < Q0; i++) area[i * 64] = quad(i);
         }
-        if (last) return;
+        __syncthreads();
+        auto finish_both = [&](int i) {
+            const float4 a = quad(i), b = area[i * 64];
+            finish(i, make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w));  // neither is -0: d starts from 0
+        };
+        if (kwi == 0) {
 #pragma unroll
-        for (int n = 0; n < N; n++) d[n] = 0.0f;
-        const int kb = kb0 + 8 * kwi + slot;
-        if (kb < nb) add_block(kb);
-        __syncthreads();  // the round's products are read
+            for (int i = 0; i < Q0; i++) finish_both(i);
+        } else {
+#pragma unroll
+            for (int i = Q0; i < Q; i++) finish_both(i);
+        }
+    } else {
+        const float4* part = lds + lane;
+        float4* mine = lds + wv * Q * 64 + lane;
+        float4* run = lds + 4 * Q * 64 + lane;
+        for (int kb0 = 32;; kb0 += 32) {
+#pragma unroll
+            for (int i = 0; i < Q; i++) mine[i * 64] = quad(i);
+            __syncthreads();
+            const bool last = !MORE || kb0 >= nb;
+            for (int i = wv; i < Q; i += 4) {
+                float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                if (MORE && kb0 > 32) s = run[i * 64];
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const float4 p = part[(j * Q + i) * 64];
+                    s = make_float4(s.x + p.x, s.y + p.y, s.z + p.z, s.w + p.w);
+                }
+                if (last)
+                    finish(i, s);
+                else
+                    run[i * 64] = s;
+            }
+            if (last) return;
+#pragma unroll
+            for (int n = 0; n < N; n++) d[n] = 0.0f;
+            const int kb = kb0 + 8 * wv + slot;
+            if (kb < nb) add_block(kb);
+            __syncthreads();  // the round's products are read
+        }
     }
 }
 
@@ -233,28 +249,29 @@ static void launch_gemv_r(const GemvCall& g, const XT* x, void* y, int ks, int k
     const int rows_wg = 4 / kw * (8 >> ks) * R;
     const unsigned grid = static_cast<unsigned>((g.rows + rows_wg - 1) / rows_wg);
     constexpr int Q = (TT * R + 3) / 4;
-    const size_t lds = kw == 1 ? 0 : static_cast<size_t>(4 + (g.nb > 8 * kw ? 4 / kw : 0)) * Q * 64 * sizeof(float4);
-    k_gemv<TYPE, TT, R, XT><<<grid, 256, lds, g.s>>>(g.w, g.rows, g.nb, g.row_stride, x, g.k, y, g.rows, g.y_bf16, ks,
-                                                   kw);
+    const bool more = g.nb > 32;
+    const size_t lds = kw == 1 ? 0 : static_cast<size_t>(kw == 2 ? 2 : more ? 5 : 4) * Q * 64 * sizeof(float4);
+    auto kernel = more ? k_gemv<TYPE, TT, R, XT, true> : k_gemv<TYPE, TT, R, XT, false>;
+    kernel<<<grid, 256, lds, g.s>>>(g.w, g.rows, g.nb, g.row_stride, x, g.k, y, g.rows, g.y_bf16, ks, kw);
 }
 
 template <int TYPE, int TT, typename XT>
 static void launch_gemv_t(const GemvCall& g, const XT* x, void* y) {
     const int ks = g.nb > 4 ? 3 : g.nb > 2 ? 2 : g.nb > 1 ? 1 : 0;
-    // wavefronts per row: up to 16 blocks one wavefront's two passes do where the rows alone are enough workgroups (us
-    // with 1 / 2; 8 tokens of fp32, Q4_K 8192 x 4096 20.8 / 23.6, 4096 x 2560 12.6 / 11.9)
-    const int kw = g.nb <= 8 || (g.nb <= 16 && g.rows >= 8192) ? 1 : g.nb <= 16 ? 2 : 4;
-    const int per_r = 4 / kw * (8 >> ks);  // rows of a workgroup per R
-    // rows per lane group: more reuse each x read, fewer leave more workgroups. Two from 256 workgroups on (us with 1 /
-    // 2 / 4 rows; 8 tokens of bf16, Q4_K 2048 x 2048 6.6 / 5.5 / 7.2, 1024 x 2048 4.8 / 5.4 / 7.1). Four from 256 on
-    // where x is read most (8 tokens of fp32, Q4_K 4096 x 2048 17.1 / 10.7 / 8.3; bf16, 2048 x 4096 11.1 / 9.2 / 8.6),
-    // else from 512 (bf16, 2 tokens, 4096 x 2048 5.0 / 4.5 / 4.9; 8 tokens, 8192 x 2048 18.7 / 14.8 / 11.5), and for
-    // one token of bf16 from 1024 (8192 x 2048 6.1 / 5.1 / 5.3, 151936 x 2048 71 / 55 / 46). One token and Q6_K
-    // never: its raw blocks fill the registers (8192 x 4096 9.2 / 8.5 / 9.1).
+    const int kw = g.nb <= 8 ? 1 : g.nb <= 16 ? 2 : 4;
+    // Rows per lane group, by the workgroups that one row each would make: more rows reuse each x read, fewer leave
+    // more workgroups (us with 1 / 2 / 4 rows below; workgroups in brackets). fp32 x: one workgroup to a CU, so two
+    // rows above 256 and four above 512 (Q4_K, 8 tokens, 1500 x 2048 [375] 9.7 / 6.7 / 7.7, 3000 x 1536 [750] 12.1
+    // / 9.5 / 7.6); one token reads x least, four above 1536 (4096 x 2048 [1024] 4.85 / 4.18 / 4.14, 6000 x 2048
+    // [1500] 5.9 / 4.9 / 5.3, 151936 x 2048 84 / 52 / 48). bf16 x, half the reads: two above 256 and four above
+    // 1536 (3 tokens, 2048 x 2048 [512] 4.4 / 4.0 / 4.5, 6000 x 2048 7.9 / 6.3 / 6.6, 8192 x 2048 [2048] 9.4 / 7.4
+    // / 6.8), with 7 and 8 tokens four above 512 (3000 x 1536 8.1 / 8.1 / 7.2), and for one token two above 1024,
+    // four above 3072 (4096 x 2048 4.21 / 4.10 / 4.13, 6000 x 2048 4.8 / 4.7 / 5.2, 151936 x 2048 68 / 50 / 43).
+    const int64_t wgs = g.rows / (4 / kw * (8 >> ks));
     constexpr bool kBf16 = sizeof(XT) == 2;
-    const int64_t least4 = TT == 1 ? (kBf16 ? 1024 : 512) : TT == 2 || (kBf16 && kw != 2) ? 512 : 256;
-    const bool four = !(TT == 1 && TYPE == WL_TYPE_Q6_K) && g.rows >= 4 * per_r * least4;
-    const int want = four ? 4 : g.rows >= 2 * per_r * 256 ? 2 : 1;
+    constexpr int kTwo = kBf16 ? (TT == 1 ? 1024 : TT < 7 ? 256 : 512) : 256;
+    constexpr int kFour = kBf16 ? (TT == 1 ? 3072 : TT < 7 ? 1536 : 512) : TT == 1 ? 1536 : 512;
+    const int want = wgs > kFour ? 4 : wgs > kTwo ? 2 : 1;
     if (want == 4)
         launch_gemv_r<TYPE, TT, 4>(g, x, y, ks, kw);
     else if (want == 2)
