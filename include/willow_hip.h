@@ -73,7 +73,8 @@ int wl_gemv(int type, const void* w, int64_t rows, int64_t k, int64_t row_stride
 
 /* wl_gemv with x and y each fp32 or bf16 (WL_DTYPE_*): bf16 values of x are read as they are, y is the fp32 sum
  * rounded to nearest even when it is bf16. What the Metal gemv takes and returns (gguf/metal.py:189-215,327-334),
- * without a conversion pass on either side. */
+ * without a conversion pass on either side. Sums are fp32, of exact weights, in wl_gemv_batch's order: a row's product
+ * has the same bits there and here, for any number of tokens, and x may be as small as fp32 holds. */
 int wl_gemv_dtype(int type, const void* w, int64_t rows, int64_t k, int64_t row_stride, const void* x, int x_dtype,
                   int64_t tokens, void* y, int y_dtype, void* stream);
 

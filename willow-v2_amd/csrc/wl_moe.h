@@ -100,8 +100,8 @@ struct PrefillArgs {
     int64_t ldo;             // o16's row stride in values
     uint16_t* o_sh16;        // [T, H] bf16
     int H, inter, sh_inter, E, k;
-    int nslab_gate_up;       // 128-row slabs of the widest intermediate dim
-    int down_slabs;          // 256-row slabs per down workgroup
+    int nslab_gate_up;       // a workgroup's slabs of the widest intermediate dim (128 rows; 64 with small tiles)
+    int down_slabs;          // slabs per down workgroup (256 rows; 128 with small tiles)
     int dense_tokens;        // > 0: k_gemm_down runs one matrix (down) over this many tokens, tiles implied
     const uint32_t* skip;    // in a fork scope: nonzero when the wait for the grouping gave up (the kernel returns)
 };

@@ -279,8 +279,8 @@ __global__ __launch_bounds__(64 * kRsWaves) void k_router_parts(const float* __r
         for (int i = 0; i < 4; i++) {
             const int f = lane + 64 * i, rr = f >> 4, c4 = 4 * (f & 15);
             const int t = t0 + rr, r = r0 + rr;
-            xn[i] = *reinterpret_cast<const float4*>(x + static_cast<int64_t>(t < T ? t : T - 1) * H + seg * kRouterSeg +
-                                                     c4);
+            xn[i] = *reinterpret_cast<const float4*>(x + static_cast<int64_t>(t < T ? t : T - 1) * H +
+                                                     seg * kRouterSeg + c4);
             const float* wr = r < rows ? (r < E ? w + static_cast<int64_t>(r) * H : shared_gate) : nullptr;
             wn[i] = wr ? *reinterpret_cast<const float4*>(wr + seg * kRouterSeg + c4) : make_float4(0.f, 0.f, 0.f, 0.f);
         }
@@ -645,7 +645,9 @@ __device__ __forceinline__ void sort_small(const int32_t* __restrict__ ids, int 
         // Few pairs (batched decode): every MFMA expert and the shared expert fit one tile of either list, so
         // the four scans below (positions, GEMV experts, the two tile lists) are one scan of three packed counts:
         // pairs in bits 0..10 (<= 1024), GEMV experts in 11..19 and MFMA experts in 20..28 (<= 256 each), whose
-        // prefix sums stay inside their fields. The same outputs, with 4 barriers instead of 13.
+        // prefix sums stay inside their fields. The same outputs, with 4 barriers instead of 13. (65 to 128 tokens on
+        // 64-token tiles take the scans below: counting tiles here instead of experts measured the same, 112 tokens
+        // 300.5 and 303 us.)
         const bool big = to.tiles && c > to.gemv_max;  // an MFMA expert
         const bool act = c > 0 && !big;                 // a GEMV expert
         int total;
@@ -1404,11 +1406,11 @@ static dim3 router_parts_grid(const WlMoeLayer& L, int64_t T) {
                 static_cast<unsigned>((nseg + kRsWaves - 1) / kRsWaves));
 }
 
-// Whether k_router_parts also normalizes a pre-norm call's rows: while a CU has at most two rows' sums of squares to
-// take one after another, counting a wavefront's rows (two from 9 tokens on) times the rounds of workgroups (82 KiB of
-// LDS, one to a CU). Layer us as its own launch / in the router: hidden 2048, 256 experts, 48 tokens (204 workgroups) 207 /
-// 207, 56 (272) 215 / 222; hidden 4096, 512 experts, 8 tokens (264) 96 / 81, 16 tokens (264) 118 / 122, 48 tokens (792)
-// 184 / 219.
+// Whether k_router_parts also normalizes a pre-norm call's rows: while a CU has at most two rows' sums of squares
+// to take one after another, counting a wavefront's rows (two from 9 tokens on) times the rounds of workgroups (82
+// KiB of LDS, one to a CU). Layer us as its own launch / in the router: hidden 2048, 256 experts, 48 tokens (204
+// workgroups) 207 / 207, 56 (272) 215 / 222; hidden 4096, 512 experts, 8 tokens (264) 96 / 81, 16 tokens (264) 118
+// / 122, 48 tokens (792) 184 / 219.
 static bool norm_in_router(const WlMoeLayer& L, int64_t T) {
     if (!router_parts(T)) return false;
     const dim3 g = router_parts_grid(L, T);
@@ -1541,8 +1543,9 @@ static int launch_router_parts(const WlMoeLayer& L, const float* x, int64_t T, c
                                bool norm, hipStream_t s) {
     const float* shared_gate = (L.shared_gate_up && L.shared_gate) ? L.shared_gate : nullptr;
     auto kernel = norm ? k_router_parts<true> : k_router_parts<false>;
-    kernel<<<router_parts_grid(L, T), 64 * kRsWaves, 0, s>>>(x, L.router, shared_gate, static_cast<int>(T), L.hidden, L.n_experts, w.parts,
-                                          xb, w.sync + kTopkDone, NormIn{L.norm_weight, L.norm_eps, w.xn});
+    kernel<<<router_parts_grid(L, T), 64 * kRsWaves, 0, s>>>(
+        x, L.router, shared_gate, static_cast<int>(T), L.hidden, L.n_experts, w.parts, xb, w.sync + kTopkDone,
+        NormIn{L.norm_weight, L.norm_eps, w.xn});
     return launch_status();
 }
 
@@ -1583,7 +1586,8 @@ static int launch_topk_parts(const WlMoeLayer& L, int64_t T, const Workspace& w,
 static int launch_sort(const WlMoeLayer& L, const Workspace& w, const int32_t* ids, int64_t T, bool tiles,
                        int gemv_max, bool fork, bool withhold, hipStream_t s) {
     const int E = L.n_experts, k = L.top_k;
-    const TileOut to{tiles ? w.tiles : nullptr, w.tiles_down, w.n_tiles, L.shared_gate_up ? 1 : 0, gemv_max, tile_caps(L, T)};
+    const TileOut to{tiles ? w.tiles : nullptr, w.tiles_down, w.n_tiles, L.shared_gate_up ? 1 : 0, gemv_max,
+                     tile_caps(L, T)};
     const int nchunks = static_cast<int>((T + kSortChunk - 1) / kSortChunk);
     if (nchunks == 1) {
         k_sort_small<<<1, kSortSmallThreads, 0, s>>>(ids, static_cast<int>(T), k, E, w.offsets, w.active, w.sorted,

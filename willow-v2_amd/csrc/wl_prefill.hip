@@ -11,8 +11,10 @@
 //   (sort)           the sort's single-workgroup stage writes the tile lists (tile_list): per-expert tiles of
 //                    sorted positions, then the shared expert's, of at most 144 (gate_up) and 128 (down) tokens,
 //                    or of 64 for both when the experts average no more (tile_caps)
-//   k_gemm_gate_up   per (tile, 128 intermediate rows; 64 with small tiles): gate and up rows together, epilogue h = silu(g) * u -> bf16
-//   k_gemm_down      per (tile, 256 output rows; 128 with small tiles): o = down h, fp32, by sorted position (combined by k_combine)
+//   k_gemm_gate_up   per (tile, 128 intermediate rows; 64 with small tiles): gate and up rows together, epilogue
+//                    h = silu(g) * u -> bf16
+//   k_gemm_down      per (tile, 256 output rows; 128 with small tiles): o = down h, bf16, by sorted position
+//                    (combined by k_combine)
 //
 // MFMA 16x16x32 bf16 operand layout (wave64): lane l holds A[l % 16][8 (l / 16) + i], B[8 (l / 16) + i][l % 16],
 // and C[4 (l / 16) + i][l % 16], i < 8 (A, B) or < 4 (C). A wavefront covers kRT row tiles x up to 9 token tiles.
@@ -845,8 +847,8 @@ static unsigned linear_grid(int nslab, int64_t tokens, int cap) {
     return static_cast<unsigned>(tiles >= kXcds ? nslab * round_up8(tiles) : round_up8(nslab) * tiles);
 }
 
-// gate_up: slab = 128-row slab of the intermediate dim; wavefront w: gate rows j0 + 16r + lr (r < kRT / 2)
-// and the matching up rows inter + j0 + ... (r >= kRT / 2), j0 = 128 slab + 8 kRT w. Epilogue h = silu(g) * u -> bf16.
+// gate_up: a slab is kSlab rows of the intermediate dim; wavefront w: gate rows j0 + 16r + lr (r < kRT / 2) and the
+// matching up rows inter + j0 + ... (r >= kRT / 2), j0 = kSlab slab + 8 kRT w. Epilogue h = silu(g) * u -> bf16.
 // TILE is tile_caps().gate_up: kTileTokens, kDownTileTokens for Q6_K rows (whose larger row state leaves no registers
 // for a ninth token tile), or kSmallTileTokens, whose slabs are 64 rows.
 template <int TYPE, int TILE>
@@ -894,8 +896,9 @@ __global__ __launch_bounds__(64 * gemm_wg_waves<TILE>(), TILE == kSmallTileToken
     gemm_tile<TYPE, TILE>(bufs, acc, nb, 1, count, a.xb, a.H, src_row, row_ptr, epi);
 }
 
-// down: a workgroup takes a.down_slabs consecutive 256-row slabs (128 with small tiles) of the hidden dim (one pipeline across them); for
-// slab item, wavefront w has rows 256 (slab0 + item) + 16 kRT w + 16 r + lr. o by position (row stride a.ldo;
+// down: a workgroup takes a.down_slabs consecutive slabs of kRows rows (256; 128 with small tiles) of the hidden dim
+// (one pipeline across them); for slab item, wavefront w has rows kRows (slab0 + item) + 16 kRT w + 16 r + lr. o by
+// position (row stride a.ldo;
 // the shared expert's by token, stride H), rounded to bf16 as the reference's bf16 F.linear output is
 // (gguf/metal.py:407). Its tiles hold at most 128 tokens (8 token tiles of accumulators keep Q6_K's wavefronts
 // within 256 registers).
@@ -974,7 +977,8 @@ __device__ __forceinline__ void gemm_ksplit(uint8_t* lds, floatx4 (&acc)[kRT][kK
     const int nphase = (nblocks + KQ - 1) / KQ;  // the last phase may hold fewer chunks
     RowState<TYPE> rs[kRT], nx[kRT];
 #pragma unroll
-    for (int r = 0; r < kRT; r++) rs[r].fetch(row_ptr(r, lr) + static_cast<int64_t>(min(kq, nblocks - 1)) * BlockInfo<TYPE>::bytes, q);
+    for (int r = 0; r < kRT; r++)
+        rs[r].fetch(row_ptr(r, lr) + static_cast<int64_t>(min(kq, nblocks - 1)) * BlockInfo<TYPE>::bytes, q);
     bf16x8 a0[kRT], a1[kRT], b[NT];
     for (int p = 0; p < nphase; p++) {
         if (p > 0) __syncthreads();  // every wavefront is done with the previous phase's chunks
@@ -1172,8 +1176,15 @@ int max_tiles(const WlMoeLayer& L, int64_t T, int cap, int gemv_max) {
     return static_cast<int>(routed + shared);
 }
 
-// The most tokens an expert averages for the small tiles. Q4_K / Q6_K layer, 256 experts, us with small / large tiles:
-// 1000 tokens (31 each) 294 / 399, 1500 315 / 410, 2000 (62) 406 / 459, 2800 (87) 486 / 485, 4096 (128) 618 / 520.
+// The most tokens an expert averages for the small tiles. Q4_K / Q6_K layer, 256 experts, uniform routing, us with
+// small / large tiles: 1000 tokens (31 each) 294 / 399, 1500 315 / 410, 2000 (62) 406 / 459, 2800 (87) 486 / 485,
+// 4096 (128) 618 / 520; of 336 shapes (16 to 256 experts, both types, 256 to 768 intermediate rows) none takes more
+// than 1.03 of the large tiles' time. The average says nothing about skew, and an expert of hundreds of tokens is
+// decoded twice as often. With popularity falling as rank^-1.1 (8 draws each) Q4_K gate_up rows still gain or tie
+// (300 tokens 148 / 159, 500 175 / 175, 1000 256 / 263, 1400 346 / 336, 1800 412 / 407) but Q6_K ones, whose decode
+// costs more, lose up to 9 % at 300 to 550 and 1200 to 1800 tokens (500 tokens 216 / 198, 1400 397 / 375), 14 % at
+// worst (128 experts, top-4, 1200 tokens), and gain 2 to 8 % at 600 to 900 (uniform: 500 tokens 321 / 374, 1000 345
+// / 443). A choice by the counts needs both kernels launched, one of them empty, for what is 2 % on average.
 constexpr int64_t kSmallTileAvg = 64;
 
 // 256-row slabs per down workgroup: several when there are enough tiles to fill the GPU with fewer workgroups, so

@@ -8,10 +8,11 @@
 namespace wl {
 
 // ---------------------------------------------------------------------------------------------------------------
-// Dequantization: one lane per (row, block, lane-chunk); each lane writes its two runs of 16 values. What bounds it is
-// the memory traffic and one trip through it (Q4_K 8192 x 2048 to bf16: 9.4 MB in, 33.6 MB out, 9.6 us = 4.5 TB/s; before 10.1). Dense rows need
-// no row index (a 64-bit division a lane), and finite scales give finite values, which v_cvt_pk_bf16_f32 rounds as
-// f32_to_bf16_bits does (a NaN would keep its payload there instead of becoming 0x7FC0).
+// Dequantization: one lane per (row, block, lane-chunk); each lane writes its two runs of 16 values. What bounds it
+// is the memory traffic and one trip through it (Q4_K 8192 x 2048 to bf16: 9.4 MB in, 33.6 MB out, 9.6 us = 4.5
+// TB/s; before 10.1). Dense rows need no row index (a 64-bit division a lane), and finite scales give finite
+// values, which v_cvt_pk_bf16_f32 rounds as f32_to_bf16_bits does (a NaN would keep its payload there instead of
+// becoming 0x7FC0).
 typedef float DequantFloat2 __attribute__((ext_vector_type(2)));
 typedef __bf16 DequantBf16x2 __attribute__((ext_vector_type(2)));
 template <bool FINITE>

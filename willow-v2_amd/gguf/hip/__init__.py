@@ -90,8 +90,8 @@ def library() -> ctypes.CDLL:
     lib.wl_moe_workspace_status.argtypes, lib.wl_moe_workspace_status.restype = [vp, ctypes.c_size_t, vp], c_int
     lib.wl_moe_fork_begin.argtypes, lib.wl_moe_fork_begin.restype = [vp], c_int
     lib.wl_moe_fork_end.argtypes, lib.wl_moe_fork_end.restype = [vp], c_int
-    for name in ("wl_dequant", "wl_gemv", "wl_gemv_dtype", "wl_linear", "wl_gemv_batch", "wl_gemv_combine", "wl_moe_check",
-                 "wl_moe_route", "wl_moe_layer", "wl_moe_layer_profile"):
+    for name in ("wl_dequant", "wl_gemv", "wl_gemv_dtype", "wl_linear", "wl_gemv_batch", "wl_gemv_combine",
+                 "wl_moe_check", "wl_moe_route", "wl_moe_layer", "wl_moe_layer_profile"):
         getattr(lib, name).restype = c_int
     _lib = lib
     return lib
@@ -252,8 +252,10 @@ class GGMLWeight:
     so each call is the same bf16 F.linear on the same values, the library GEMM alone. With keep_dense False nothing
     is kept between calls: each call is the reference's own form, the weight dequantized to a bf16 temporary and
     the library GEMM on it (bit for bit the reference's arithmetic). linear_mfma (wl_linear, the weights dequantized
-    in registers, no temporary) is the form for a caller that cannot hold the temporary; on dense shapes it is the
-    slower one at every token count measured from 16 to 8192."""
+    in registers, no temporary; its sums in another order) is the form for a caller that cannot hold the temporary. It
+    is the faster one of the two up to some hundreds of tokens (Q4_K 4096x2048 up to 1000: 12.9 against 24.7 us at 200,
+    28.6 against 33.3 at 1000; Q6_K 2048x2048 up to 512), the slower one above (45.7 against 40.3 us at 4096, Q4_K
+    2048x2048), and slower throughout where few rows meet a long k (256x16384)."""
 
     keep_dense = True
 
